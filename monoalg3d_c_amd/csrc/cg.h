@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "cg_resident.h"
 #include "mono_common.h"
 #include "operator.h"
 
@@ -86,6 +87,17 @@ class CgWorkspace {
     // CSR variant (non-uniform meshes), FP64.
     int solve_csr(const CsrMatrix &A, const double *b, double *x, const CgConfig &cfg, CgStats *st, hipStream_t s);
 
+    // Solves as one launch each (cg_resident.h).  resident_begin says whether
+    // the operator's solves run that way, and makes room for `count` of them;
+    // resident_enqueue puts one on the stream; resident_finish waits for those
+    // enqueued and returns the device's record, its totals those since the last
+    // resident_finish (`stop` is cleared for the next ones).  op32 null: FP64 CG.
+    bool resident_begin(const OpView<double> &op64, const OpView<float> *op32, const CgConfig &cfg, int count, hipStream_t s, int *rc);
+    int resident_enqueue(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x, const CgConfig &cfg,
+                         hipStream_t s);
+    int resident_finish(ResidentStatus *out, hipStream_t s);
+    const int32_t *resident_stop() const { return rst ? &rst->stop : nullptr; }
+
     int64_t n = 0;
     // FP64 vectors
     double *r = nullptr, *p = nullptr, *p2 = nullptr, *q = nullptr, *z = nullptr;
@@ -115,7 +127,7 @@ class CgWorkspace {
     // gaps are ~1% of a 16M-cell step and ~3.5% of a batch step), and the
     // replays measured 0.4% (16M cells) to 2% (batch) slower.
     struct PrefixKey {
-        int kind = 0;  // 0 FP64, 1 mixed
+        int kind = 0;  // 0 FP64, 1 mixed, 2 FP64 in one launch, 3 mixed in one launch
         std::vector<int> sched;
         OpView<double> op64{};
         OpView<float> op32{};
@@ -138,7 +150,18 @@ class CgWorkspace {
     // has been seen before; returns 0 or -1 (HIP error).
     template <class F> int run_prefix(const PrefixKey &key, hipStream_t s, int &state, F &&enqueue);
 
+    ResidentPlan rplan[2];            // FP64, mixed
+    ResidentStatus *rst = nullptr;    // device
+    ResidentStatus *host_rst = nullptr;  // pinned mirror
+    ResidentStatus rst_seen{};           // the record at the last resident_finish
+    uint64_t resident_epochs = 0;     // bound on the exchanges since the last reset
+    bool use_resident = true;         // MONO_RESIDENT=0 in the environment at init: never
+    int resident_pause = 0;           // after a time-out: solves left to the kernels of cg.hip
+    int resident_backoff = 0;
+
   private:
+    int solve_one_resident(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x, const CgConfig &cfg,
+                           CgStats *st, hipStream_t s);
     int fp64_launches(const OpView<double> &op, const double *b, double *x, const CgConfig &cfg, int k0, int count, int &nres,
                       hipStream_t s);
 };

@@ -1238,6 +1238,13 @@ int CgWorkspace::init(int64_t n_, int64_t, bool fp32) {
     MONO_CHECK(hipHostMalloc(&host_sc, 2 * sizeof(CgScalars), hipHostMallocDefault));
     MONO_CHECK(hipMalloc(&sweep_its, sizeof(int) * kMaxBlindSweeps));
     MONO_CHECK(hipHostMalloc(&host_its, sizeof(int) * kMaxBlindSweeps, hipHostMallocDefault));
+    MONO_CHECK(hipMalloc(&rst, sizeof(ResidentStatus)));
+    MONO_CHECK(hipMemset(rst, 0, sizeof(ResidentStatus)));
+    MONO_CHECK(hipHostMalloc(&host_rst, sizeof(ResidentStatus), hipHostMallocDefault));
+    const char *ur = getenv("MONO_RESIDENT"), *uw = getenv("MONO_RESIDENT_WAIT_US");
+    use_resident = !(ur && ur[0] == '0');
+    if(uw)
+        for(ResidentPlan &rp : rplan) rp.wait_ticks = (uint64_t)atoll(uw) * 100;
     const char *ug = getenv("MONO_GRAPH");
     use_graphs = ug && ug[0] == '1';
     return 0;
@@ -1258,6 +1265,11 @@ int CgWorkspace::release() {
     for(PrefixGraph &g : graphs)
         if(g.exec) MONO_CHECK(hipGraphExecDestroy(g.exec));
     graphs.clear();
+    for(ResidentPlan &rp : rplan)
+        if(resident_release(&rp)) return -1;
+    if(rst) MONO_CHECK(hipFree(rst));
+    if(host_rst) MONO_CHECK(hipHostFree(host_rst));
+    rst = host_rst = nullptr;
     sweep_its = nullptr;
     host_its = nullptr;
     last_sched.clear();
@@ -1432,8 +1444,96 @@ int CgWorkspace::fp64_launches(const OpView<double> &op, const double *b, double
     return 0;
 }
 
+bool CgWorkspace::resident_begin(const OpView<double> &op64, const OpView<float> *op32, const CgConfig &cfg, int count, hipStream_t s,
+                                 int *rc) {
+    *rc = 0;
+    if(!rst || !use_resident || cfg.jacobi || cfg.poll_chunk > 0 || count < 1) return false;
+    if(resident_pause > 0) {
+        resident_pause--;
+        return false;
+    }
+    // exchanges a solve may need; their 32-bit numbers start again long before they run out
+    const uint64_t most = op32 ? ((uint64_t)cfg.max_its + 3) * ((uint64_t)cfg.max_outer + 1) : (uint64_t)cfg.max_its + 2;
+    if(cfg.max_its < 0 || cfg.max_outer < 0 || most > (1ull << 30) / (unsigned)count) return false;
+    ResidentPlan &p = rplan[op32 ? 1 : 0];
+    if(resident_plan(&p, op64, op32, cfg)) {
+        *rc = -1;
+        return false;
+    }
+    if(p.state != 1) return false;
+    if(resident_epochs + most * (unsigned)count > (1ull << 31)) {
+        if(resident_reset(rplan, 2, rst, s)) {
+            *rc = -1;
+            return false;
+        }
+        resident_epochs = 0;
+    }
+    resident_epochs += most * (unsigned)count;
+    return true;
+}
+
+int CgWorkspace::resident_enqueue(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x, const CgConfig &cfg,
+                                  hipStream_t s) {
+    const ResidentPlan &p = rplan[op32 ? 1 : 0];
+    auto launch = [&]() -> int { return resident_launch(p, op64, op32, b, x, cfg, rst, s); };
+    if(!use_graphs) return launch();
+    PrefixKey key;
+    key.kind = op32 ? 3 : 2;
+    key.op64 = op64;
+    if(op32) key.op32 = *op32;
+    key.b = b;
+    key.x = x;
+    key.cfg = cfg;
+    int no_state = 0;
+    return run_prefix(key, s, no_state, launch);
+}
+
+int CgWorkspace::resident_finish(ResidentStatus *out, hipStream_t s) {
+    MONO_CHECK(hipMemcpyAsync(host_rst, rst, sizeof(ResidentStatus), hipMemcpyDeviceToHost, s));
+    MONO_CHECK(hipStreamSynchronize(s));
+    *out = *host_rst;
+    out->solves -= rst_seen.solves;
+    out->cg_total -= rst_seen.cg_total;
+    out->inner_total -= rst_seen.inner_total;
+    out->outer_total -= rst_seen.outer_total;
+    rst_seen = *host_rst;
+    if(out->stop != kResidentGoing) {
+        if(resident_reset(rplan, 2, rst, s)) return -1;
+        resident_epochs = 0;
+        if(out->stop == kResidentTimeout) {
+            // the chip is shared with launches of the same kind: leave it to
+            // the others for a while, each time for longer
+            resident_backoff = resident_backoff < 1024 ? 4 * resident_backoff + 16 : resident_backoff;
+            resident_pause = resident_backoff;
+        }
+    }
+    return 0;
+}
+
+// 0: solved, 1: the launch gave up (x is a valid start), -1: error
+int CgWorkspace::solve_one_resident(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x,
+                                    const CgConfig &cfg, CgStats *st, hipStream_t s) {
+    if(resident_enqueue(op64, op32, b, x, cfg, s)) return -1;
+    ResidentStatus r;
+    if(resident_finish(&r, s)) return -1;
+    if(r.stop == kResidentTimeout) return 1;
+    if(st) {
+        st->iterations = r.last_its;
+        st->error = r.last_err;
+        st->outer = r.last_outer;
+        st->inner_total = r.last_its - 1;
+    }
+    return 0;
+}
+
 int CgWorkspace::solve_fp64(const OpView<double> &op, const double *b, double *x, const CgConfig &cfg, CgStats *st, hipStream_t s) {
     if(check_pattern(op.pat)) return -1;
+    int rrc = 0;
+    if(resident_begin(op, nullptr, cfg, 1, s, &rrc)) {
+        const int rc = solve_one_resident(op, nullptr, b, x, cfg, st, s);
+        if(rc <= 0) return rc;
+    }
+    if(rrc) return -1;
     int nres = 0;
     auto iterations = [&](int k0, int count) -> int { return fp64_launches(op, b, x, cfg, k0, count, nres, s); };
     // the last solve's iteration count includes the kernel that detected
@@ -1470,6 +1570,12 @@ int CgWorkspace::solve_mixed(const OpView<double> &op64, const OpView<float> &op
                              CgStats *st, hipStream_t s) {
     const int grid = grid_for(op64.n);
     if(check_pattern(op64.pat)) return -1;
+    int rrc = 0;
+    if(resident_begin(op64, &op32, cfg, 1, s, &rrc)) {
+        const int rc = solve_one_resident(op64, &op32, b, x, cfg, st, s);
+        if(rc <= 0) return rc;
+    }
+    if(rrc) return -1;
     float *pb[2] = {p32, p32b};
     int inner_total = 0, corrections = 0;
     int chunk0 = last_inner > 2 ? last_inner + 1 : 4;

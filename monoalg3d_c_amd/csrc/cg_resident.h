@@ -1,0 +1,67 @@
+// Whole diffusion solve in one launch (host interface of cg_resident.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "mono_common.h"
+#include "operator.h"
+
+namespace mono {
+
+struct CgConfig;
+
+// Device record of the resident solves on one workspace.  The kernels of a
+// step do nothing while `stop` is set, so solves can be enqueued ahead of the
+// host's look at it.
+enum ResidentStop : int32_t {
+    kResidentGoing = 0,
+    kResidentNan = 1,      // the last solve ended with r.r = NaN (it is counted)
+    kResidentTimeout = 2,  // a block waited too long for another: the solve is not done
+};
+struct ResidentStatus {
+    int32_t stop;
+    uint32_t epoch;        // exchanges done so far on this workspace
+    int64_t solves;        // solves completed
+    int64_t cg_total;      // sum of the reference's iteration counts
+    int64_t inner_total;   // CG iterations run
+    int64_t outer_total;   // outer sweeps
+    int32_t last_its;
+    int32_t last_outer;
+    double last_err;
+};
+
+// One block's share of the box and how many blocks there are.
+struct ResidentGeom {
+    int bx, by, bz;     // cells of a tile
+    int tx, ty, tz;     // tiles
+    int rpt;            // cells per thread
+    int threads;
+    int halo;           // most halo cells of a tile
+    size_t lds;
+    bool cooperative;
+};
+
+// Buffers of the resident solves of one workspace.
+struct ResidentPlan {
+    int state = 0;               // 0 not planned, 1 usable, -1 not for this operator
+    // what the plan was made for
+    int nx = 0, ny = 0, nz = 0, pat = 0, mode = 0, mixed = -1;
+    ResidentGeom g{};
+    unsigned long long *words = nullptr;  // exchanged values of both parities
+    unsigned long long *sums = nullptr;   // partial sums of both parities
+    uint64_t wait_ticks = 2000000;  // longest wait of a block for another: 20 ms of the 100 MHz clock
+    size_t words_bytes = 0;
+    size_t sums_bytes = 0;
+};
+
+// Decide the tiles for an operator and make the buffers (p->state).
+int resident_plan(ResidentPlan *p, const OpView<double> &op64, const OpView<float> *op32, const CgConfig &cfg);
+int resident_release(ResidentPlan *p);
+// Enqueues the solve; op32 null: FP64 CG.
+int resident_launch(const ResidentPlan &p, const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x,
+                    const CgConfig &cfg, ResidentStatus *st, hipStream_t s);
+// Clears the exchange buffers and the epoch (and `stop`) on the stream.
+int resident_reset(const ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s);
+
+}  // namespace mono

@@ -32,6 +32,9 @@ template <typename T> struct IonicLaunch {
     int first_step;         // read V from sv row 0 instead of v (t = 0: no Vm mirror)
     int block;              // step kernels: threads per block (0: the built-in choice)
     int write_vm_row;       // also store V* in sv row 0
+    // if set and not 0 on the device: do nothing (a solve enqueued before this
+    // launch has stopped the run)
+    const int32_t *stop;
     // adaptive Euler (launch_ionic_adaptive): per-cell dt, time_new and
     // previous_dt in three FP64 rows of `pitch`; each cell advances from its
     // time_new to final_time

@@ -112,6 +112,7 @@ __device__ __forceinline__ void ionic_step_body(const IonicLaunch<T> &a, const f
     // range), and its right-hand side is 0.
     bool live = true;
     if constexpr(ACT) live = a.active[i] != 0;
+    const int stop = a.stop ? *a.stop : 0;
 
     T y[NEQ];
 #pragma unroll
@@ -124,6 +125,7 @@ __device__ __forceinline__ void ionic_step_body(const IonicLaunch<T> &a, const f
     } else {
         V = a.first_step ? (double)a.sv[i] : stream_load(&a.v[i]);
     }
+    if(stop) return;
 
     const double st = live ? cell_stim(a, i) : 0.0;
     if constexpr(ONE && MODEL == kORd2011) {
@@ -171,6 +173,7 @@ __device__ __forceinline__ void adaptive_body(const IonicLaunch<T> &a) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= a.n) return;
     if(a.active && !a.active[i]) return;
+    if(a.stop && *a.stop) return;
     T y[NEQ], k1[NEQ], k2[NEQ], yp[NEQ];
 #pragma unroll
     for(int s = 1; s < NEQ; s++) y[s] = a.sv[(size_t)s * a.pitch + i];

@@ -631,6 +631,7 @@ static OpView<T> make_view(const Operator &o, const T *table, const T *tint, con
     v.nz = o.nz;
     v.n = o.n;
     v.pat = o.pat;
+    v.full_pat = o.full_pat;
     v.table = table;
     v.table_int = tint;
     v.percell = percell;
@@ -743,6 +744,7 @@ int build_operator(const AssemblyParams &p, const double *coef27, Operator *op, 
     op->nslots = (int)slots.size();
     std::vector<int> bslots;  // the smallest pattern covering every row (per-cell storage order)
     const int pb = choose_pattern(slots, &bslots);
+    op->full_pat = pb;
 
     // class table candidate: representative cell of each (z, cy, cx) class
     const int ncls = p.nz * 9;

@@ -519,6 +519,7 @@ static int launch_ionic(mono_tissue *t, double stim_amp, int block) {
         a.dt = t->dt_ode;
         a.num_steps = t->num_ode_steps;
         a.first_step = t->st.steps == 0;
+        a.stop = t->cg.resident_stop();
         a.block = block;
         if(d.ode_adaptive) {
             set_adaptive(t, a);
@@ -547,6 +548,7 @@ static int launch_ionic(mono_tissue *t, double stim_amp, int block) {
         a.dt = (float)t->dt_ode;
         a.num_steps = t->num_ode_steps;
         a.first_step = t->st.steps == 0;
+        a.stop = t->cg.resident_stop();
         a.block = block;
         if(d.ode_adaptive) {
             set_adaptive(t, a);
@@ -656,70 +658,174 @@ static int tuned_block(mono_tissue *t, bool &timed) {
     return u.cand[u.pending];
 }
 
+// The stimulus amplitude of the step that begins at the tissue's time (merged
+// stimulus, ode_solver.c:288-341: inclusive window on the accumulated time,
+// summed over the ODE sub-steps); moves a periodic stimulus on.
+static double step_stimulus(mono_tissue *t) {
+    const mono_tissue_desc &d = t->d;
+    double amp = 0.0;
+    double tt = t->cur_time;
+    for(int j = 0; j < t->num_ode_steps; j++) {
+        if((tt >= t->stim_start) && (tt <= t->stim_start + d.stim_duration)) amp += d.stim_current;
+        tt += t->dt_ode;
+    }
+    // the shifted start goes back into the configuration as "%lf" text and
+    // is parsed again (ode_solver.c:224-230): it keeps six decimals
+    if(d.stim_period > 0.0 && tt >= t->stim_start + d.stim_period) {
+        char buf[64];
+        snprintf(buf, sizeof(buf), "%lf", t->stim_start + d.stim_period);
+        t->stim_start = strtod(buf, nullptr);
+    }
+    return amp;
+}
+
+// Enqueue the step's ionic launch (and the batch's tolerance kernels).
+static int enqueue_ionic(mono_tissue *t) {
+    const double amp = step_stimulus(t);
+    bool tuned = false;
+    const int block = tuned_block(t, tuned);
+    if(block < 0) return -1;
+    if(tuned) MONO_CHECK(hipEventRecord(t->tune.e0, t->stream));
+    if(t->timing) MONO_CHECK(hipEventRecord(t->ev[0], t->stream));
+    if(launch_ionic(t, amp, block)) return -1;
+    if(t->timing) MONO_CHECK(hipEventRecord(t->ev[1], t->stream));
+    if(tuned) MONO_CHECK(hipEventRecord(t->tune.e1, t->stream));
+    if(t->tol_dev && launch_instance_tolerance(t)) return -1;
+    return 0;
+}
+
+// Solve the step's system and wait for it.
+static int solve_step(mono_tissue *t, CgStats *cs) {
+    // the Jacobi update reads each row's diagonal from the stored rows, so a
+    // preconditioned FP64 solve keeps them (mask-mode views store none)
+    if(t->d.precision == MONO_FP64)
+        return t->cg.solve_fp64(t->cgcfg.jacobi ? t->op.view64() : t->op.view64_solve(), t->b, t->v, t->cgcfg, cs, t->stream);
+    return t->cg.solve_mixed(t->op.view64_solve(), t->op.view32(), t->b, t->v, t->cgcfg, cs, t->stream);
+}
+
+// Time and counters at the end of a step.
+static void end_step(mono_tissue *t) {
+    t->st.steps++;
+    t->cur_time += t->d.dt_pde;
+    t->st.time = t->cur_time;
+}
+static void count_solve(mono_tissue *t, const CgStats &cs) {
+    t->st.cg_iterations_total += cs.iterations;
+    t->st.last_cg_iterations = cs.iterations;
+    t->st.last_cg_error = cs.error;
+    t->st.last_outer = cs.outer;
+    t->st.inner_iterations_total += cs.inner_total;
+    t->st.outer_sweeps_total += cs.outer;
+}
+
+}  // extern "C"
+
+// One step after the other, each solve waited for.
+static int step_waiting(mono_tissue *t) {
+    if(enqueue_ionic(t)) return -1;
+    CgStats cs{};
+    if(solve_step(t, &cs)) return -1;
+    if(t->timing) {
+        MONO_CHECK(hipEventRecord(t->ev[2], t->stream));
+        MONO_CHECK(hipEventSynchronize(t->ev[2]));
+        float a = 0, b = 0;
+        MONO_CHECK(hipEventElapsedTime(&a, t->ev[0], t->ev[1]));
+        MONO_CHECK(hipEventElapsedTime(&b, t->ev[1], t->ev[2]));
+        t->st.ionic_ms_total += a;
+        t->st.solve_ms_total += b;
+    }
+    count_solve(t, cs);
+    end_step(t);
+    if(isnan(cs.error)) {
+        t->st.nan_detected = 1;
+        return 1;
+    }
+    return 0;
+}
+
+// Steps enqueued without looking at their solves in between.  The host looks
+// once per kStepsAhead steps: a 65k-cell step of ~50 us would lose 15 us more to each
+// look, and the queue holds several times as many launches.
+constexpr int kStepsAhead = 256;
+
+int mono_tissue_advance(mono_tissue *t, int nsteps, const std::function<int(int)> &after) {
+    struct Clock {
+        double cur_time, stim_start;
+    };
+    std::vector<Clock> at;
+    int k = 0;
+    while(k < nsteps) {
+        int count = std::min(nsteps - k, kStepsAhead), rc = 0;
+        const bool mixed = t->d.precision != MONO_FP64;
+        const OpView<double> op64 = t->op.view64_solve();
+        const OpView<float> op32 = mixed ? t->op.view32() : OpView<float>{};
+        if(t->timing || !t->cg.resident_begin(op64, mixed ? &op32 : nullptr, t->cgcfg, count, t->stream, &rc)) {
+            if(rc) return -1;
+            const int r = step_waiting(t);
+            if(r < 0) return -1;
+            if(after && after(k)) return -1;
+            if(r == 1) return 1;
+            k++;
+            continue;
+        }
+        const mono_stats before = t->st;
+        at.clear();
+        for(int j = 0; j < count; j++) {
+            at.push_back({t->cur_time, t->stim_start});
+            if(enqueue_ionic(t)) return -1;
+            if(t->cg.resident_enqueue(op64, mixed ? &op32 : nullptr, t->b, t->v, t->cgcfg, t->stream)) return -1;
+            end_step(t);
+            if(after && after(k + j)) return -1;
+        }
+        at.push_back({t->cur_time, t->stim_start});
+        ResidentStatus r;
+        if(t->cg.resident_finish(&r, t->stream)) return -1;
+        const int done = (int)r.solves;
+        if(done > 0) {
+            t->st.cg_iterations_total += r.cg_total;
+            t->st.inner_iterations_total += r.inner_total;
+            t->st.outer_sweeps_total += r.outer_total;
+            t->st.last_cg_iterations = r.last_its;
+            t->st.last_cg_error = r.last_err;
+            t->st.last_outer = r.last_outer;
+        }
+        if(done < count || r.stop == kResidentNan) {
+            // the run stopped early: back to the clock after the last step done
+            t->st.steps = before.steps + done;
+            t->cur_time = t->st.time = at[done].cur_time;
+            t->stim_start = at[done].stim_start;
+        }
+        if(r.stop == kResidentNan) {
+            t->st.nan_detected = 1;
+            return 1;
+        }
+        k += done;
+        if(done < count) {
+            // the next step's ionic launch has run, its solve has not: solve it here
+            (void)step_stimulus(t);
+            CgStats cs{};
+            if(solve_step(t, &cs)) return -1;
+            count_solve(t, cs);
+            end_step(t);
+            if(after && after(k)) return -1;
+            if(isnan(cs.error)) {
+                t->st.nan_detected = 1;
+                return 1;
+            }
+            k++;
+        }
+    }
+    return 0;
+}
+
+extern "C" {
+
 int mono_tissue_step(mono_tissue *t, int nsteps) {
     if(!t) {
         mono_set_error("null tissue");
         return -1;
     }
-    const mono_tissue_desc &d = t->d;
-    for(int k = 0; k < nsteps; k++) {
-        // merged stimulus (ode_solver.c:288-341): inclusive window on the
-        // accumulated time, summed over the ODE sub-steps
-        double amp = 0.0;
-        double tt = t->cur_time;
-        for(int j = 0; j < t->num_ode_steps; j++) {
-            if((tt >= t->stim_start) && (tt <= t->stim_start + d.stim_duration)) amp += d.stim_current;
-            tt += t->dt_ode;
-        }
-        // the shifted start goes back into the configuration as "%lf" text and
-        // is parsed again (ode_solver.c:224-230): it keeps six decimals
-        if(d.stim_period > 0.0 && tt >= t->stim_start + d.stim_period) {
-            char buf[64];
-            snprintf(buf, sizeof(buf), "%lf", t->stim_start + d.stim_period);
-            t->stim_start = strtod(buf, nullptr);
-        }
-
-        bool tuned = false;
-        const int block = tuned_block(t, tuned);
-        if(block < 0) return -1;
-        if(tuned) MONO_CHECK(hipEventRecord(t->tune.e0, t->stream));
-        if(t->timing) MONO_CHECK(hipEventRecord(t->ev[0], t->stream));
-        if(launch_ionic(t, amp, block)) return -1;
-        if(t->timing) MONO_CHECK(hipEventRecord(t->ev[1], t->stream));
-        if(tuned) MONO_CHECK(hipEventRecord(t->tune.e1, t->stream));
-        if(t->tol_dev && launch_instance_tolerance(t)) return -1;
-        CgStats cs{};
-        int rc;
-        // the Jacobi update reads each row's diagonal from the stored rows, so a
-        // preconditioned FP64 solve keeps them (mask-mode views store none)
-        if(d.precision == MONO_FP64)
-            rc = t->cg.solve_fp64(t->cgcfg.jacobi ? t->op.view64() : t->op.view64_solve(), t->b, t->v, t->cgcfg, &cs, t->stream);
-        else rc = t->cg.solve_mixed(t->op.view64_solve(), t->op.view32(), t->b, t->v, t->cgcfg, &cs, t->stream);
-        if(rc) return -1;
-        if(t->timing) {
-            MONO_CHECK(hipEventRecord(t->ev[2], t->stream));
-            MONO_CHECK(hipEventSynchronize(t->ev[2]));
-            float a = 0, b = 0;
-            MONO_CHECK(hipEventElapsedTime(&a, t->ev[0], t->ev[1]));
-            MONO_CHECK(hipEventElapsedTime(&b, t->ev[1], t->ev[2]));
-            t->st.ionic_ms_total += a;
-            t->st.solve_ms_total += b;
-        }
-        t->st.steps++;
-        t->st.cg_iterations_total += cs.iterations;
-        t->st.last_cg_iterations = cs.iterations;
-        t->st.last_cg_error = cs.error;
-        t->st.last_outer = cs.outer;
-        t->st.inner_iterations_total += cs.inner_total;
-        t->st.outer_sweeps_total += cs.outer;
-        t->cur_time += d.dt_pde;
-        t->st.time = t->cur_time;
-        if(isnan(cs.error)) {
-            t->st.nan_detected = 1;
-            return 1;
-        }
-    }
-    return 0;
+    return mono_tissue_advance(t, nsteps, nullptr);
 }
 
 int mono_tissue_sync(mono_tissue *t) {

@@ -4,6 +4,8 @@
 
 #include <stdint.h>
 
+#include <functional>
+
 #include "../../include/monoalg_hip.h"
 #include "cg.h"
 #include "observer.h"
@@ -62,3 +64,8 @@ struct mono_tissue {
     double cur_time = 0.0;
     mono_stats st{};
 };
+
+// Advance the tissue by nsteps; after(k), if given, is called when step k has
+// been enqueued, to enqueue work on its results (again for a step that had to
+// be solved anew).  1 when a NaN stopped the run, -1 on an error.
+int mono_tissue_advance(mono_tissue *t, int nsteps, const std::function<int(int)> &after);
