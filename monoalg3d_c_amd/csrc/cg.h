@@ -21,7 +21,7 @@ namespace mono {
 // kernel, at most kMaxRed sums each, stored sum-major (sum k of block b at
 // k * kMaxBlocks + b).
 constexpr int kMaxBlocks = 8192;
-constexpr int kMaxRed = 3;
+constexpr int kMaxRed = 4;
 
 struct CsrMatrix {
     int n = 0;
@@ -29,7 +29,8 @@ struct CsrMatrix {
     const int64_t *row_ptr = nullptr;  // device
     const int32_t *col = nullptr;      // device
     const double *val = nullptr;       // device
-    const double *diag = nullptr;      // device, optional (Jacobi)
+    const int *bad = nullptr;          // device, optional: not 0: malformed, nothing is solved
+    const double *dinv = nullptr;      // device, Jacobi solves: 1 / diagonal
 };
 
 // Stopping rule: the reference's absolute test on r.r (linear_system_solver.c:95,159-163)
@@ -50,11 +51,11 @@ struct CgConfig {
     const double *tol_dev = nullptr;
 };
 
-// Device buffers of a CSR solve: r, p, q, z (n doubles each), two partial-sum
+// Device buffers of a CSR solve: r, p, s, w (n doubles each), two partial-sum
 // buffers (kMaxBlocks * kMaxRed doubles each), the device scalar record and a
 // host record the solve polls into (pinned or not).
 struct CsrBuffers {
-    double *r = nullptr, *p = nullptr, *q = nullptr, *z = nullptr;
+    double *r = nullptr, *p = nullptr, *s = nullptr, *w = nullptr;
     double *P0 = nullptr, *P1 = nullptr;
     CgScalars *sc = nullptr;
     CgScalars *host_sc = nullptr;
@@ -70,8 +71,8 @@ struct CgStats {
 // CSR conjugate gradient (FP64) on caller-provided buffers.
 int csr_solve(const CsrMatrix &A, const double *b, double *x, const CgConfig &cfg, CgStats *st, hipStream_t s,
               const CsrBuffers &w);
-// diag[i] = A(i, i) (0 where the row has no diagonal entry; the last entry wins)
-hipError_t launch_csr_diag(const CsrMatrix &A, double *diag, hipStream_t s);
+// dinv[i] = 1 / A(i, i) (1 where the row has no diagonal entry or a zero one; the last entry wins)
+hipError_t launch_csr_dinv(const CsrMatrix &A, double *dinv, hipStream_t s);
 // b[i] = alpha[i] * vm[i] (UPDATE_MONODOMAIN)
 hipError_t launch_rhs(int64_t n, const double *alpha, const double *vm, double *b, hipStream_t s);
 class CgWorkspace {

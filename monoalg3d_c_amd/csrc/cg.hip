@@ -19,14 +19,17 @@
 // Mixed precision (FP32 CG with FP64 defect correction): the outer residual
 // r = b - A x is formed in FP64 with the FP64 operator; an FP32 CG solves
 // A d = r to a relative tolerance with FP64 dot accumulation; x += d in FP64.
+#include <math.h>
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
 #include "aniso_row.h"
 #include "cg.h"
+#include "wave_sum.h"
 
 namespace mono {
 
@@ -53,34 +56,24 @@ __device__ __forceinline__ void chunk_range(int64_t n, int64_t &beg, int64_t &en
     end = beg + per < n ? beg + per : n;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for(int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    return v;
-}
-
 // Block-wide sums; the totals are returned to every thread.
 template <int NR> __device__ __forceinline__ void block_sum_all(double (&v)[NR]) {
     __shared__ double lds[NR][kBlock / 64];
-    __shared__ double tot[NR];
+    __syncthreads();  // (an earlier call's sums have been read)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    wave_sums(v);
+    if(lane == kSumLane) {
+#pragma unroll
+        for(int k = 0; k < NR; k++) lds[k][w] = v[k];
+    }
+    __syncthreads();
 #pragma unroll
     for(int k = 0; k < NR; k++) {
-        const double s = wave_sum(v[k]);
-        if(lane == 0) lds[k][w] = s;
-    }
-    __syncthreads();
-    if(threadIdx.x == 0) {
+        double s = 0.0;
 #pragma unroll
-        for(int k = 0; k < NR; k++) {
-            double s = 0.0;
-            for(int i = 0; i < kBlock / 64; i++) s += lds[k][i];
-            tot[k] = s;
-        }
+        for(int i = 0; i < kBlock / 64; i++) s += lds[k][i];
+        v[k] = s;
     }
-    __syncthreads();
-#pragma unroll
-    for(int k = 0; k < NR; k++) v[k] = tot[k];
 }
 
 // This block's contribution to the kernel's reductions.
@@ -105,6 +98,7 @@ template <int NR> __device__ __forceinline__ void write_partials_at(double (&v)[
 template <int NR> __device__ __forceinline__ void sum_partials(const double *__restrict__ P, int nprev, double (&tot)[NR]) {
 #pragma unroll
     for(int k = 0; k < NR; k++) tot[k] = 0.0;
+#pragma unroll 4
     for(int i = threadIdx.x; i < nprev; i += kBlock) {
 #pragma unroll
         for(int k = 0; k < NR; k++) tot[k] += P[k * kMaxBlocks + i];
@@ -1016,96 +1010,208 @@ __global__ void k_note_sweep(const CgScalars *si, const CgScalars *so, int *out)
 }
 
 // ---------------------------------------------------------------------------
-// CSR (non-uniform meshes), FP64: one wave per row.
+// CSR (non-uniform meshes), FP64.
+//
+// Two launches per CG iteration: the product w = A z with the iteration's sums,
+// and the update of the vectors with alpha and beta from them.  s = A p is
+// carried along (s = w + beta s), so p.s needs no pass of its own: it is
+//     p.s = z.w + beta (z.s_old + p_old.w) + beta^2 (p.s)_old
+// (for any A), and the iterates are those of the two-reduction form.  z = r, or
+// D^-1 r with Jacobi, formed where it is read (dinv: 1 / D).
+//
+// Finite-volume rows have 4 to 30 entries.  A wave per row left most of its
+// lanes without an entry (520k rows of 3M entries: 91 us, 0.6 TB/s of the 57 MB
+// that a product with its sums needs; here 14 us).  Here the entries of kBlock rows are read as one stream, every lane
+// loading the next one, their products go to LDS, and a thread adds up each
+// row there.  Row groups with a row of more than kStreamRow entries keep a wave
+// per row (a single thread would add a long row alone while the others wait;
+// at 64 entries a wave's lanes are full).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
-                                                     const double *__restrict__ val, const double *__restrict__ x,
-                                                     double *__restrict__ y, const CgScalars *sc) {
-    if(sc && sc->done) return;
-    const int lane = threadIdx.x & 63;
-    const int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
-    if(row >= n) return;
-    double acc = 0.0;
-    for(int64_t kk = rp[row] + lane; kk < rp[row + 1]; kk += 64) acc += val[kk] * x[col[kk]];
-    acc = wave_sum(acc);
-    if(lane == 0) y[row] = acc;
-}
+constexpr int kStream = 2048;    // products in LDS at a time: 7 entries per row of a block
+constexpr int kStreamRow = 64;
+constexpr int kCsrBlocks = 1024;  // most blocks of a product: every block of the update reads all their sums
 
-__global__ __launch_bounds__(kBlock) void k_csr_res(int n, const double *__restrict__ Ax, const double *__restrict__ b,
-                                                    const double *__restrict__ diag, double *__restrict__ r, double *__restrict__ p,
-                                                    double *__restrict__ z, int jacobi, double *Pout) {
-    int64_t beg, end;
-    chunk_range(n, beg, end);
-    double v[3] = {0.0, 0.0, 0.0};
-    for(int64_t c = beg + threadIdx.x; c < end; c += kBlock) {
-        const double rc = b[c] - Ax[c];
-        r[c] = rc;
-        if(jacobi) {
-            double d = diag[c];
-            if(d == 0.0) d = 1.0;
-            const double zc = (1.0 / d) * rc;
-            z[c] = zc;
-            p[c] = zc;
-            v[1] += rc * zc;
-        } else {
-            p[c] = rc;
+constexpr int kCsrSteps = 512;    // most blocks of an update
+// (3M entries, 520k rows, 17 iterations, whole solve: 509 us as 1024 and 512
+// blocks; 603 as 512 and 512; 756 as 2024 and 512, twice the sums to read)
+
+// Row sums of A u over the rows [row0, row0 + kBlock) of a block, u(c) the
+// vector's element c; the sum of row row0 + threadIdx.x is returned to its thread.
+template <class U>
+__device__ __forceinline__ double csr_rows(int n, int64_t row0, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                           const double *__restrict__ val, double *prod, U &&u) {
+    const int t = threadIdx.x, lane = t & 63;
+    const int64_t row = row0 + t;
+    const int64_t beg = rp[row < n ? row : n], end = rp[row + 1 < n ? row + 1 : n];
+    const int64_t k0 = rp[row0], k1 = rp[row0 + kBlock < n ? row0 + kBlock : n];
+    double sum = 0.0;
+    if(__syncthreads_or(end - beg > kStreamRow)) {
+        for(int i = t >> 6; i < kBlock; i += kBlock / 64) {
+            if(row0 + i >= n) break;
+            double a = 0.0;
+            for(int64_t k = rp[row0 + i] + lane; k < rp[row0 + i + 1]; k += 64) a += val[k] * u(col[k]);
+            double row_sum[1] = {a};
+            wave_sums(row_sum);
+            if(lane == kSumLane) prod[i] = row_sum[0];
         }
-        v[0] += rc * rc;
-        v[2] += b[c] * b[c];
+        __syncthreads();
+        if(row < n) sum = prod[t];
+        __syncthreads();
+        return sum;
     }
-    write_partials<3>(v, Pout);
+    for(int64_t c0 = k0; c0 < k1; c0 += kStream) {
+        const int m = (int)(k1 - c0 < kStream ? k1 - c0 : kStream);
+        constexpr int kU = 8;  // all of a block's loads in flight together
+        for(int i = t; i < m; i += kU * kBlock) {
+            int32_t cc[kU];
+            double vv[kU];
+#pragma unroll
+            for(int j = 0; j < kU; j++) {
+                const int64_t k = c0 + (i + j * kBlock < m ? i + j * kBlock : i);
+                cc[j] = col[k];
+                vv[j] = val[k];
+            }
+#pragma unroll
+            for(int j = 0; j < kU; j++) {
+                const double pr = vv[j] * u(cc[j]);
+                if(i + j * kBlock < m) prod[i + j * kBlock] = pr;
+            }
+        }
+        __syncthreads();
+        const int64_t a = beg > c0 ? beg : c0, e = end < c0 + m ? end : c0 + m;
+        for(int64_t k = a; k < e; k++) sum += prod[k - c0];
+        __syncthreads();
+    }
+    return sum;
 }
 
-// p = rz + beta p after the stopping test (prologue over the previous partials)
-__global__ __launch_bounds__(kBlock) void k_csr_dir(int n, double *__restrict__ p, const double *__restrict__ rz, CgSetup cs, int mode,
-                                                    int k, const double *Pin, int nprev, CgScalars *sc) {
-    double beta = 0.0;
-    bool now;
-    if(!iter_prologue(mode, k, Pin, nprev, sc, nullptr, cs, beta, now)) return;
-    int64_t beg, end;
-    chunk_range(n, beg, end);
-    for(int64_t c = beg + threadIdx.x; c < end; c += kBlock) p[c] = rz[c] + beta * p[c];
-}
-
-__global__ __launch_bounds__(kBlock) void k_csr_dot(int n, const double *__restrict__ p, const double *__restrict__ q, double *Pout,
-                                                    const CgScalars *sc) {
-    if(sc->done) return;
-    int64_t beg, end;
-    chunk_range(n, beg, end);
+// r = b - A x; partial b.b
+__global__ __launch_bounds__(kBlock) void k_csr_res(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                    const double *__restrict__ val, const double *__restrict__ x,
+                                                    const double *__restrict__ b, double *__restrict__ r, double *Pout, const int *bad) {
+    if(bad && *bad) return;
+    __shared__ double prod[kStream];
+    const int64_t groups = ((int64_t)n + kBlock - 1) / kBlock, per = (groups + gridDim.x - 1) / gridDim.x;
+    const int64_t g0 = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * per;
     double v[1] = {0.0};
-    for(int64_t c = beg + threadIdx.x; c < end; c += kBlock) v[0] += p[c] * q[c];
+    for(int64_t g = g0; g < g0 + per && g < groups; g++) {
+        const double ax = csr_rows(n, g * kBlock, rp, col, val, prod, [&](int32_t c) { return x[c]; });
+        const int64_t i = g * kBlock + threadIdx.x;
+        if(i < n) {
+            const double bc = b[i];
+            r[i] = bc - ax;
+            v[0] += bc * bc;
+        }
+    }
     write_partials<1>(v, Pout);
 }
 
-__global__ __launch_bounds__(kBlock) void k_csr_update(int n, double *__restrict__ x, const double *__restrict__ p,
-                                                       const double *__restrict__ q, double *__restrict__ r, double *__restrict__ z,
-                                                       const double *__restrict__ diag, int jacobi, int k, const double *Pin, int nprev,
-                                                       double *Pout, CgScalars *sc) {
-    if(sc->done) return;
-    double pq[1];
-    sum_partials<1>(Pin, nprev, pq);
-    const double a = sc->rrs[k & 1] / pq[0];
-    if(blockIdx.x == 0 && threadIdx.x == 0) {
-        sc->pAp = pq[0];
-        sc->alpha = a;
+// w = A z; partials r.r, r.z, z.w, z.s + p.w (the last only after the first iteration)
+template <bool JACOBI>
+__global__ __launch_bounds__(kBlock) void k_csr_mult(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                     const double *__restrict__ val, const double *__restrict__ r,
+                                                     const double *__restrict__ dinv, const double *__restrict__ p,
+                                                     const double *__restrict__ s, double *__restrict__ w, int k, double *Pout,
+                                                     const CgScalars *sc, const int *bad) {
+    if(k > 0 ? sc->done : (bad && *bad)) return;
+    __shared__ double prod[kStream];
+    const int64_t groups = ((int64_t)n + kBlock - 1) / kBlock, per = (groups + gridDim.x - 1) / gridDim.x;
+    const int64_t g0 = (int64_t)xcd_chunk(blockIdx.x, gridDim.x) * per;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for(int64_t g = g0; g < g0 + per && g < groups; g++) {
+        const double az = csr_rows(n, g * kBlock, rp, col, val, prod, [&](int32_t c) { return JACOBI ? dinv[c] * r[c] : r[c]; });
+        const int64_t i = g * kBlock + threadIdx.x;
+        if(i < n) {
+            const double rc = r[i], zc = JACOBI ? dinv[i] * rc : rc;
+            w[i] = az;
+            v[0] += rc * rc;
+            v[1] += rc * zc;
+            v[2] += zc * az;
+            if(k > 0) v[3] += zc * s[i] + p[i] * az;
+        }
     }
+    write_partials<4>(v, Pout);
+}
+
+// Iteration k with the sums of k_csr_mult: the stopping test on r (and before
+// the first iteration the tolerance, from the residual's b.b), beta, alpha;
+//     p = z + beta p, s = w + beta s, x += alpha p, r -= alpha s
+// The scalars of the previous iteration are read from the record's other slot,
+// which this kernel does not write.
+template <bool JACOBI>
+__global__ __launch_bounds__(kBlock) void k_csr_step(int n, double *__restrict__ x, double *__restrict__ p, double *__restrict__ s,
+                                                     const double *__restrict__ w, double *__restrict__ r,
+                                                     const double *__restrict__ dinv, int k, const double *Pin, int nprev,
+                                                     const double *Pres, CgSetup cs, CgScalars *sc, const int *bad) {
+    if(k == 0 && bad && *bad) {
+        if(blockIdx.x == 0 && threadIdx.x == 0) {
+            sc->done_iter = -1;
+            sc->done = 1;
+        }
+        return;
+    }
+    __shared__ int s_done;
+    if(threadIdx.x == 0) s_done = k > 0 && sc->done && sc->done_iter < k;
+    __syncthreads();
+    if(s_done) return;
+    double t[4];
+    sum_partials<4>(Pin, nprev, t);
+    const double rr = t[0], rz = t[1];
+    double tol = sc->tol_abs;
+    if(k == 0) {
+        double bb[1];
+        sum_partials<1>(Pres, nprev, bb);
+        tol = cs.rel_tol > 0.0 ? cs.rel_tol * cs.rel_tol * bb[0] : cs.tol;
+    }
+    const int iters = 1 + k;
+    const bool done = k == 0 ? (!(rr >= tol) || cs.max_its <= 1) : (rr <= tol || iters >= cs.max_its || rr != rr);
+    const double beta = k == 0 ? 0.0 : rz / sc->rrs[(k - 1) & 1];
+    const double ps = t[2] + beta * (t[3] + beta * (k == 0 ? 0.0 : sc->pqs[(k - 1) & 1]));
+    const double alpha = rz / ps;
+    if(blockIdx.x == 0 && threadIdx.x == 0) {
+        if(k == 0) {
+            sc->tol_abs = tol;
+            sc->rr0 = rr;
+            sc->max_its = cs.max_its;
+            sc->done_iter = 0x7fffffff;
+        }
+        sc->rrs[k & 1] = rz;
+        sc->pqs[k & 1] = ps;
+        sc->rr_true = rr;
+        sc->iters = iters;
+        sc->beta = beta;
+        sc->alpha = alpha;
+        if(done) {
+            sc->done_iter = k;
+            __threadfence();
+        }
+        sc->done = done;
+    }
+    if(done) return;
     int64_t beg, end;
     chunk_range(n, beg, end);
-    double v[2] = {0.0, 0.0};
-    for(int64_t c = beg + threadIdx.x; c < end; c += kBlock) {
-        x[c] += a * p[c];
-        const double rc = r[c] - a * q[c];
-        r[c] = rc;
-        if(jacobi) {
-            double d = diag[c];
-            if(d == 0.0) d = 1.0;
-            const double zc = (1.0 / d) * rc;
-            z[c] = zc;
-            v[1] += zc * rc;
+    for(int64_t c0 = beg + threadIdx.x; c0 < end; c0 += kIlp * kBlock) {
+        double pv[kIlp], sv[kIlp], wv[kIlp], rv[kIlp], xv[kIlp];
+#pragma unroll
+        for(int u = 0; u < kIlp; u++) {
+            const int64_t c = c0 + u * kBlock < end ? c0 + u * kBlock : c0;
+            pv[u] = k == 0 ? 0.0 : p[c];
+            sv[u] = k == 0 ? 0.0 : s[c];
+            wv[u] = w[c];
+            rv[u] = r[c];
+            xv[u] = x[c];
         }
-        v[0] += rc * rc;
+#pragma unroll
+        for(int u = 0; u < kIlp; u++) {
+            const int64_t c = c0 + u * kBlock;
+            if(c >= end) continue;
+            const double pn = (JACOBI ? dinv[c] * rv[u] : rv[u]) + beta * pv[u], sn = wv[u] + beta * sv[u];
+            p[c] = pn;
+            s[c] = sn;
+            x[c] = xv[u] + alpha * pn;
+            r[c] = rv[u] - alpha * sn;
+        }
     }
-    write_partials<2>(v, Pout);
 }
 
 // ---------------------------------------------------------------------------
@@ -1700,8 +1806,8 @@ int CgWorkspace::solve_csr(const CsrMatrix &A, const double *b, double *x, const
     CsrBuffers w;
     w.r = r;
     w.p = p;
-    w.q = q;
-    w.z = z;
+    w.s = p2;
+    w.w = q;
     w.P0 = P0;
     w.P1 = P1;
     w.sc = sc;
@@ -1710,29 +1816,38 @@ int CgWorkspace::solve_csr(const CsrMatrix &A, const double *b, double *x, const
 }
 
 int csr_solve(const CsrMatrix &A, const double *b, double *x, const CgConfig &cfg, CgStats *st, hipStream_t s, const CsrBuffers &w) {
-    const int grid = grid_for(A.n);
-    const unsigned sgrid = (unsigned)(((int64_t)A.n * 64 + kBlock - 1) / kBlock);
+    const int grid = std::min(kCsrSteps, grid_for(A.n));
+    const int64_t groups = ((int64_t)A.n + kBlock - 1) / kBlock, per = (groups + kCsrBlocks - 1) / kCsrBlocks;
+    int mgrid = (int)((groups + per - 1) / per);
+    if(mgrid >= 64) mgrid = (mgrid + 7) / 8 * 8;  // whole rounds of the XCD order; at most kCsrBlocks
     const CgSetup cs{cfg.tol, cfg.rel_tol, cfg.inner_rel, cfg.max_its, cfg.jacobi, cfg.max_outer, 0, nullptr};
-    double *r = w.r, *p = w.p, *q = w.q, *z = w.z, *P0 = w.P0, *P1 = w.P1;
     CgScalars *sc = w.sc, *host_sc = w.host_sc;
-    k_csr_spmv<<<sgrid, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, x, q, nullptr);
-    k_csr_res<<<grid, kBlock, 0, s>>>(A.n, q, b, A.diag, r, p, z, cfg.jacobi, P0);
+    k_csr_res<<<mgrid, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, x, b, w.r, w.P1, A.bad);
     MONO_CHECK(hipGetLastError());
-    const double *rz = cfg.jacobi ? z : r;
     int enq = 0;
-    int chunk = cfg.poll_chunk > 0 ? cfg.poll_chunk : 4;
+    // iterations between looks at the record: eight, then as many as the
+    // residual's fall so far says are left (a look costs as much as several
+    // iterations, and so do a few that find the solve done)
+    int chunk = cfg.poll_chunk > 0 ? cfg.poll_chunk : 8;
     for(;;) {
         for(int j = 0; j < chunk; j++) {
             const int k = enq + j;
-            k_csr_dir<<<grid, kBlock, 0, s>>>(A.n, p, rz, cs, k == 0 ? 0 : 1, k, P0, grid, sc);
-            k_csr_spmv<<<sgrid, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, p, q, sc);
-            k_csr_dot<<<grid, kBlock, 0, s>>>(A.n, p, q, P1, sc);
-            k_csr_update<<<grid, kBlock, 0, s>>>(A.n, x, p, q, r, z, A.diag, cfg.jacobi, k, P1, grid, P0, sc);
+            if(cfg.jacobi) {
+                k_csr_mult<true><<<mgrid, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, w.r, A.dinv, w.p, w.s, w.w, k, w.P0, sc, A.bad);
+                k_csr_step<true><<<grid, kBlock, 0, s>>>(A.n, x, w.p, w.s, w.w, w.r, A.dinv, k, w.P0, mgrid, w.P1, cs, sc, A.bad);
+            } else {
+                k_csr_mult<false><<<mgrid, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, w.r, nullptr, w.p, w.s, w.w, k, w.P0, sc, A.bad);
+                k_csr_step<false><<<grid, kBlock, 0, s>>>(A.n, x, w.p, w.s, w.w, w.r, nullptr, k, w.P0, mgrid, w.P1, cs, sc, A.bad);
+            }
         }
         MONO_CHECK(hipGetLastError());
         enq += chunk;
         if(poll(sc, host_sc, s)) return -1;
         if(host_sc->done || enq > cfg.max_its + 2) break;
+        if(cfg.poll_chunk <= 0) {
+            const double fell = log(host_sc->rr0 / host_sc->rr_true) / (enq - 1), left = log(host_sc->rr_true / host_sc->tol_abs);
+            chunk = fell > 0.0 && left / fell < 15.0 ? 1 + (int)(left / fell) : 16;
+        }
     }
     if(st) {
         st->iterations = host_sc->iters;
@@ -1743,19 +1858,21 @@ int csr_solve(const CsrMatrix &A, const double *b, double *x, const CgConfig &cf
     return 0;
 }
 
-__global__ __launch_bounds__(kBlock) void k_csr_diag(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
-                                                     const double *__restrict__ val, double *__restrict__ diag) {
+// 1 / A(i, i), 1 where the row has no diagonal entry or a zero one
+__global__ __launch_bounds__(kBlock) void k_csr_dinv(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                     const double *__restrict__ val, const int *bad, double *__restrict__ dinv) {
+    if(bad && *bad) return;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if(i >= n) return;
     double d = 0.0;
     for(int64_t k = rp[i]; k < rp[i + 1]; k++)
         if(col[k] == (int32_t)i) d = val[k];
-    diag[i] = d;
+    dinv[i] = 1.0 / (d == 0.0 ? 1.0 : d);
 }
 
-hipError_t launch_csr_diag(const CsrMatrix &A, double *diag, hipStream_t s) {
+hipError_t launch_csr_dinv(const CsrMatrix &A, double *dinv, hipStream_t s) {
     const unsigned g = (unsigned)(((int64_t)A.n + kBlock - 1) / kBlock);
-    k_csr_diag<<<g, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, diag);
+    k_csr_dinv<<<g, kBlock, 0, s>>>(A.n, A.row_ptr, A.col, A.val, A.bad, dinv);
     return hipGetLastError();
 }
 

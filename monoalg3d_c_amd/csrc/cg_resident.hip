@@ -56,6 +56,7 @@
 #include <algorithm>
 
 #include "cg.h"
+#include "wave_sum.h"
 
 namespace mono {
 
@@ -76,31 +77,8 @@ __device__ __forceinline__ void put_value(u64 *w, uint32_t epoch, double v) {
     word_store(w + 1, tagged(epoch, (uint32_t)(bits >> 32)));
 }
 
-// Sums over the wave, in its last lane (DPP row shifts and broadcasts; fixed
-// order).  Step by step over all sums, so each hides the others' latency.
 constexpr int kSums = 3;       // sums of an exchange
 constexpr int kSumWords = 8;   // words of a block's sums (two each, to a whole number of 64 bytes)
-template <int CTRL, int ROWS> __device__ __forceinline__ void dpp_plus(double (&v)[kSums]) {
-    double u[kSums];
-#pragma unroll
-    for(int k = 0; k < kSums; k++) {
-        const u64 bits = (u64)__double_as_longlong(v[k]);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)bits, CTRL, ROWS, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(bits >> 32), CTRL, ROWS, 0xf, false);
-        u[k] = __longlong_as_double((long long)(((u64)(uint32_t)hi << 32) | (uint32_t)lo));
-    }
-#pragma unroll
-    for(int k = 0; k < kSums; k++) v[k] += u[k];
-    __builtin_amdgcn_sched_barrier(0);
-}
-__device__ __forceinline__ void wave_totals(double (&v)[kSums]) {
-    dpp_plus<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
-    dpp_plus<0x112, 0xf>(v);
-    dpp_plus<0x114, 0xf>(v);
-    dpp_plus<0x118, 0xf>(v);
-    dpp_plus<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    dpp_plus<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-}
 
 struct ResidentArgs {
     OpView<double> op64;
@@ -410,8 +388,8 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                     if(two) sum[k] += join(h[6 + 2 * k], h[7 + 2 * k]);
                 }
             }
-            wave_totals(sum);
-            if(lane == 63) {
+            wave_sums(sum);
+            if(lane == kSumLane) {
 #pragma unroll
                 for(int k = 0; k < kSums; k++) part[kSums * NW + k] = sum[k];
             }
@@ -458,8 +436,8 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             if((mask >> (16 + q)) & 1u) put_value(W + (size_t)kWords<T2> * ((size_t)blockIdx.x * (RPT * T) + local(q)), epoch, value(q));
             breathe<RPT == 16, 4>(q);
         }
-        wave_totals(t);
-        if(lane == 63) {
+        wave_sums(t);
+        if(lane == kSumLane) {
 #pragma unroll
             for(int k = 0; k < kSums; k++) part[k * NW + wave] = t[k];
         }

@@ -25,7 +25,7 @@ struct mono_csr {
     int64_t *row_ptr = nullptr;
     int32_t *col = nullptr;
     double *val = nullptr;
-    double *diag = nullptr;
+    double *dinv = nullptr;   // 1 / diagonal
     double *b = nullptr;      // right-hand side (uploaded, or formed by mono_csr_update_rhs)
     double *x = nullptr;      // warm start / solution
     double *vm = nullptr;     // mono_csr_update_rhs: uploaded Vm
@@ -60,7 +60,7 @@ static int check_csr(const char *who, int n, const int64_t *row_ptr, const int32
 // mono_cg_csr_device_noalloc: the CSR solve of mono_cg_csr on operands the
 // caller already holds on the device, with every buffer of the solve in one
 // fixed area of device memory that the library reserves at load time, so that
-// a call allocates nothing.  Layout (doubles): diagonal, r, p, q, z (n each,
+// a call allocates nothing.  Layout (doubles): 1 / diagonal, r, p, s, w (n each,
 // n <= kNoAllocMaxRows), two partial-sum areas (kMaxBlocks * kMaxRed each),
 // the scalar record, then the operand check's verdict.  Each device holds its
 // own copy of the area; concurrent calls on one device share it and race.
@@ -117,6 +117,9 @@ __global__ void k_csr_check_rows(int n, const int64_t *__restrict__ rp, int *ver
     if(bad) atomicOr(verdict, bad);
 }
 __global__ void k_csr_check_cols(int n, const int64_t *__restrict__ rp, const int32_t *__restrict__ col, int *verdict) {
+    // after a malformed row_ptr nothing is read through it (block 0 of this very
+    // kernel may set bit 3 already)
+    if(verdict[0] & 7) return;
     const int64_t nnz = rp[n];
     for(int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nnz; k += (int64_t)gridDim.x * blockDim.x)
         if(col[k] < 0 || col[k] >= n) {
@@ -151,36 +154,22 @@ int mono_cg_csr_device_noalloc(int n, const int64_t *row_ptr, const int32_t *col
     int *verdict = (int *)(base + kNoAllocCheckOff);
     k_clear_verdict<<<1, 64, 0, s>>>(verdict);
     k_csr_check_rows<<<(unsigned)((n + 1 + 255) / 256), 256, 0, s>>>(n, row_ptr, verdict);
-    MONO_CHECK(hipGetLastError());
-    int flags = 0;
-    MONO_CHECK(hipMemcpyAsync(&flags, verdict, sizeof(int), hipMemcpyDeviceToHost, s));
-    MONO_CHECK(hipStreamSynchronize(s));
-    if(flags) {
-        mono_set_error("%s: malformed row_ptr (%s%s%s)", who, flags & 1 ? "row_ptr[0] != 0 " : "",
-                       flags & 2 ? "decreasing entries " : "", flags & 4 ? "row_ptr[n] < 0" : "");
-        return -1;
-    }
     k_csr_check_cols<<<1024, 256, 0, s>>>(n, row_ptr, col, verdict);
     MONO_CHECK(hipGetLastError());
-    MONO_CHECK(hipMemcpyAsync(&flags, verdict, sizeof(int), hipMemcpyDeviceToHost, s));
-    MONO_CHECK(hipStreamSynchronize(s));
-    if(flags) {
-        mono_set_error("%s: column index out of range", who);
-        return -1;
-    }
     double *v = (double *)base;
     CsrMatrix M;
     M.n = n;
     M.row_ptr = row_ptr;
     M.col = col;
     M.val = val;
-    M.diag = v;
-    MONO_CHECK(launch_csr_diag(M, v, s));
+    M.dinv = v;
+    M.bad = verdict;  // the solve's kernels look at it before they read through the operands
+    if(jacobi) MONO_CHECK(launch_csr_dinv(M, v, s));
     CsrBuffers w;
     w.r = v + kNoAllocMaxRows;
     w.p = v + 2 * kNoAllocMaxRows;
-    w.q = v + 3 * kNoAllocMaxRows;
-    w.z = v + 4 * kNoAllocMaxRows;
+    w.s = v + 3 * kNoAllocMaxRows;
+    w.w = v + 4 * kNoAllocMaxRows;
     w.P0 = (double *)(base + 5 * kNoAllocVecBytes);
     w.P1 = (double *)(base + 5 * kNoAllocVecBytes + kNoAllocPartBytes);
     w.sc = (CgScalars *)(base + kNoAllocScOff);
@@ -191,7 +180,18 @@ int mono_cg_csr_device_noalloc(int n, const int64_t *row_ptr, const int32_t *col
     cfg.jacobi = jacobi;
     CgStats st{};
     if(csr_solve(M, b, x, cfg, &st, s, w)) return -1;
+    int flags = 0;
+    MONO_CHECK(hipMemcpyAsync(&flags, verdict, sizeof(int), hipMemcpyDeviceToHost, s));
     MONO_CHECK(hipStreamSynchronize(s));
+    if(flags & 7) {
+        mono_set_error("%s: malformed row_ptr (%s%s%s)", who, flags & 1 ? "row_ptr[0] != 0 " : "",
+                       flags & 2 ? "decreasing entries " : "", flags & 4 ? "row_ptr[n] < 0" : "");
+        return -1;
+    }
+    if(flags) {
+        mono_set_error("%s: column index out of range", who);
+        return -1;
+    }
     if(iterations) *iterations = st.iterations;
     if(error) *error = st.error;
     return 0;
@@ -202,7 +202,7 @@ int mono_csr_destroy(mono_csr *A) {
     int rc = 0;
     if(A->stream && hipStreamSynchronize(A->stream) != hipSuccess) rc = -1;
     if(A->ws.release()) rc = -1;
-    void *bufs[] = {A->row_ptr, A->col, A->val, A->diag, A->b, A->x, A->vm, A->alpha};
+    void *bufs[] = {A->row_ptr, A->col, A->val, A->dinv, A->b, A->x, A->vm, A->alpha};
     for(void *p : bufs)
         if(p && hipFree(p) != hipSuccess) rc = -1;
     if(A->stream && hipStreamDestroy(A->stream) != hipSuccess) rc = -1;
@@ -233,7 +233,7 @@ int mono_csr_create(int n, const int64_t *row_ptr, const int32_t *col, const dou
     if(e == hipSuccess) e = hipMalloc(&A->row_ptr, sizeof(int64_t) * (n + 1));
     if(e == hipSuccess) e = hipMalloc(&A->col, sizeof(int32_t) * nz);
     if(e == hipSuccess) e = hipMalloc(&A->val, sizeof(double) * nz);
-    if(e == hipSuccess) e = hipMalloc(&A->diag, sizeof(double) * n);
+    if(e == hipSuccess) e = hipMalloc(&A->dinv, sizeof(double) * n);
     if(e == hipSuccess) e = hipMalloc(&A->b, sizeof(double) * n);
     if(e == hipSuccess) e = hipMalloc(&A->x, sizeof(double) * n);
     if(e == hipSuccess) e = hipMemcpyAsync(A->row_ptr, row_ptr, sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice, A->stream);
@@ -248,7 +248,7 @@ int mono_csr_create(int n, const int64_t *row_ptr, const int32_t *col, const dou
     M.row_ptr = A->row_ptr;
     M.col = A->col;
     M.val = A->val;
-    e = launch_csr_diag(M, A->diag, A->stream);
+    e = launch_csr_dinv(M, A->dinv, A->stream);
     if(e == hipSuccess) e = hipStreamSynchronize(A->stream);
     if(e != hipSuccess) return fail(e);
     if(A->ws.init(n, n, false)) {
@@ -318,7 +318,7 @@ int mono_csr_solve(mono_csr *A, const double *b, double *x, double tol, int max_
     M.row_ptr = A->row_ptr;
     M.col = A->col;
     M.val = A->val;
-    M.diag = A->diag;
+    M.dinv = A->dinv;
     CgConfig cfg;
     cfg.tol = tol;
     cfg.max_its = max_its;

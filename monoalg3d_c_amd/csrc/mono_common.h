@@ -42,6 +42,7 @@ struct CgScalars {
     double rrs[2];    // r.z (r.r without Jacobi) by iteration parity
     double rr_true;   // r.r of the current residual (stopping test, reported error)
     double pAp;
+    double pqs[2];    // CSR solves: p.Ap by iteration parity
     double alpha;
     double beta;
     double rr0;       // r.r at the start of the solve
