@@ -6,11 +6,11 @@
 // 27-bit mask: bit slot_of(ox, oy, oz) is set when the neighbour at that
 // offset lies in the box and is active, bit 13 when the cell itself is active.
 // With per-layer (or uniform) tensors and no per-cell conductivity factor the
-// row depends on nothing else, so the stencil kernels can form it on the fly
-// from 4 bytes per cell instead of reading 27 stored coefficients.  In FP64
-// the operations are those of k_assemble in the same order (both files build
-// with FMA contraction off), and the operator builder checks the two bit for
-// bit before it hands the mask to a kernel.
+// row depends on nothing else, so the stencil kernels can apply it from 4 bytes
+// per cell (mask_aniso_apply) instead of reading 27 stored coefficients.
+// mask_aniso_row forms the row: in FP64 with the operations of k_assemble in
+// the same order (both files build with FMA contraction off), and the operator
+// builder checks the two bit for bit before it hands the mask to a kernel.
 //
 // Reference rule: calc_sigmas / fill_elements_aniso (assembly_common.c:115-830),
 // anisotropic_sigma_assembly_matrix (matrix_assembly.c:389-514).
@@ -284,7 +284,9 @@ __host__ __device__ __forceinline__ void mask_assemble_fast(const T (&h)[kNDir],
 }
 
 // FAST: the flux sigmas by mask_flux_fast and the coefficients by
-// mask_assemble_fast; otherwise the operations of k_assemble in its order.
+// mask_assemble_fast (what a kernel that needs the coefficients themselves
+// would use; checked on the host); otherwise the operations of k_assemble in
+// its order.
 template <typename T, bool FAST = false>
 __host__ __device__ __forceinline__ void mask_aniso_row(uint32_t m, const T (&tz)[3][6], T dx, T dy, T dz, T alpha, T (&row)[27]) {
 #pragma unroll
@@ -555,6 +557,157 @@ __host__ __device__ __forceinline__ void mask_aniso_row(uint32_t m, const T (&tz
     row[13] = diag;
 #pragma unroll
     for(int d = 0; d < kNDir; d++) row[dir_slot(d)] = acc[d];
+}
+
+// ---------------------------------------------------------------------------
+// The row applied to the values around the cell, without forming it.
+//
+// The flux through face (a, s) has a normal part, w (u_C - u_N), and for each
+// of the two other axes b a tangential part: minus s X times the sum over the
+// face's neighbour pairs straddling it along b (offsets 0 and s along a, -1..1
+// along the third axis c) of u(+b) - u(-b), where both cells are there.  X is
+// the cross conductivity averaged over those pairs and divided by their count
+// once more, times half the length the flux is integrated over; 0 where the
+// face's neighbour is missing.  The product with the row is then 27 masked
+// differences, the sums of them that the faces share, and 12 weights X.
+// A weight depends on the layer and on which of six pairs are there, so it is
+// read from a table of its layer (kMaskTable entries, staged in LDS by the
+// kernels).  VALU issue bounds the mask sweep: about 350 instructions a row in
+// FP32, staging and epilogue included, where forming the 26 coefficients (with
+// their averages and reciprocals) and multiplying by them took 640.  400x400x50
+// cells, 10% of them inactive: FP32 sweep 160 -> 89 us (33 us of memory
+// traffic), FP64 residual 223 -> 126 us; 203x151x40: FP64 sweep 48 -> 30 us.
+//
+// Table of a layer, by pair direction b and flux axis a:
+//   kXY0: b = x, a = y;  kXY1: b = y, a = x: by the six pairs' bits (mask_fold);
+//   kXZ:  b = x, a = z;  kYZ:  b = y, a = z: [s > 0][4 n0 + n1], n0 pairs in the
+//         cell's layer and n1 in the neighbour's;
+//   kZX:  b = z, a = x;  kZY:  b = z, a = y: by the number of pairs;
+//   kNormal: the faces' normal weights w: x, y, z - 1, z + 1.
+// ---------------------------------------------------------------------------
+enum MaskTable { kXY0 = 0, kXY1 = 64, kXZ = 128, kYZ = 160, kZX = 192, kZY = 200, kNormal = 208, kMaskTable = 256 };
+
+// v where `keep` is all ones, 0 where it is 0
+__host__ __device__ __forceinline__ float mask_keep(float v, int32_t keep) {
+    return __builtin_bit_cast(float, __builtin_bit_cast(int32_t, v) & keep);
+}
+__host__ __device__ __forceinline__ double mask_keep(double v, int32_t keep) {
+    struct Halves {
+        int32_t lo, hi;
+    } h = __builtin_bit_cast(Halves, v);
+    h.lo &= keep;
+    h.hi &= keep;
+    return __builtin_bit_cast(double, h);
+}
+// all ones where bit k of m is set (hidden from the device compiler, which
+// otherwise makes a compare and two selects of each masked FP64 value)
+__host__ __device__ __forceinline__ int32_t mask_ones(uint32_t m, int k) {
+    int32_t r = (int32_t)(m << (31 - k)) >> 31;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+v"(r));
+#endif
+    return r;
+}
+
+// The pairs are named by the slot of their lower cell.  Bits of the six pairs
+// of flux axis x or y (two offsets along it, three layers), moved to bits 0..5:
+// lower offset and layer l at `first` + 9 l, upper offset `step` above.
+template <int STEP> __host__ __device__ __forceinline__ int mask_fold(uint32_t avail, int first) {
+    static_assert(STEP == 1 || STEP == 3, "offset along x or y");
+    constexpr int k = STEP == 1 ? 7 : 8;  // layers fold to bits {0,1} {2,3} {4,5}, or {0,3} {1,4} {2,5}
+    constexpr uint32_t six = (1u << 0 | 1u << STEP) * (1u | 1u << 9 | 1u << 18);
+    const uint32_t t = (avail >> first) & six;
+    return (int)((t | t >> k | t >> (2 * k)) & 63u);
+}
+
+// The table of layer z: lt = the tensors (xx yy zz xy xz yz) of layers z - 1,
+// z, z + 1, clamped at the ends.
+inline void mask_layer_table(const double *const (&lt)[3], double dx, double dy, double dz, double *out) {
+    for(int i = 0; i < kMaskTable; i++) out[i] = 0.0;
+    for(int i = 1; i < 64; i++) {
+        double s0 = 0.0, s1 = 0.0;
+        for(int l = 0; l < 3; l++) {
+            s0 += lt[l][3] * ((i >> l & 1) + (i >> (l + 3) & 1));
+            s1 += lt[l][3] * ((i >> (2 * l) & 1) + (i >> (2 * l + 1) & 1));
+        }
+        const double np = __builtin_popcount(i);
+        out[kXY0 + i] = 0.5 * dz * s0 / (np * np);
+        out[kXY1 + i] = 0.5 * dz * s1 / (np * np);
+    }
+    for(int up = 0; up < 2; up++)
+        for(int n0 = 0; n0 < 4; n0++)
+            for(int n1 = n0 == 0 ? 1 : 0; n1 < 4; n1++) {
+                const double np = n0 + n1;
+                const double *nb = lt[up ? 2 : 0];
+                out[kXZ + 16 * up + 4 * n0 + n1] = 0.5 * dy * (n0 * lt[1][4] + n1 * nb[4]) / (np * np);
+                out[kYZ + 16 * up + 4 * n0 + n1] = 0.5 * dx * (n0 * lt[1][5] + n1 * nb[5]) / (np * np);
+            }
+    for(int np = 1; np <= 6; np++) {
+        out[kZX + np] = 0.25 * dy * (lt[2][4] + lt[0][4]) / np;
+        out[kZY + np] = 0.25 * dx * (lt[2][5] + lt[0][5]) / np;
+    }
+    out[kNormal + 0] = lt[1][0] * ((dy * dz) / dx);
+    out[kNormal + 1] = lt[1][1] * ((dx * dz) / dy);
+    out[kNormal + 2] = 0.5 * (lt[0][2] + lt[1][2]) * ((dx * dy) / dz);
+    out[kNormal + 3] = 0.5 * (lt[2][2] + lt[1][2]) * ((dx * dy) / dz);
+}
+
+// Row of a cell with mask m times the values u(slot).  w: the normal weights,
+// xt: the layer's table; diag, if given, gets the row's diagonal.
+template <typename T, class U>
+__host__ __device__ __forceinline__ T mask_aniso_apply(uint32_t m, const T (&w)[4], T alpha, const T *xt, U &&u, double *diag = nullptr) {
+    const int32_t lx = mask_ones(m, 12), rx = mask_ones(m, 14), ly = mask_ones(m, 10), ry = mask_ones(m, 16), lz = mask_ones(m, 4),
+                  rz = mask_ones(m, 22);
+    const T a0 = mask_keep(alpha, mask_ones(m, 13));
+    const T uc = u(13);
+    const T wlx = mask_keep(w[0], lx), wrx = mask_keep(w[0], rx), wly = mask_keep(w[1], ly), wry = mask_keep(w[1], ry),
+            wlz = mask_keep(w[2], lz), wrz = mask_keep(w[3], rz);
+    T acc = a0 * uc;
+    acc += wlx * (uc - u(12)) + wrx * (uc - u(14));
+    acc += wly * (uc - u(10)) + wry * (uc - u(16));
+    acc += wlz * (uc - u(4)) + wrz * (uc - u(22));
+    if(diag) *diag = (double)(a0 + ((wlx + wrx) + (wly + wry) + (wlz + wrz)));
+    {  // pairs along x at (y, z)
+        const uint32_t av = m & (m >> 2);
+        T d[3][3];
+#pragma unroll
+        for(int z = 0; z < 3; z++)
+#pragma unroll
+            for(int y = 0; y < 3; y++) d[y][z] = mask_keep(u(3 * y + 9 * z + 2) - u(3 * y + 9 * z), mask_ones(av, 3 * y + 9 * z));
+        const T y0 = (d[0][0] + d[0][1]) + d[0][2], y1 = (d[1][0] + d[1][1]) + d[1][2], y2 = (d[2][0] + d[2][1]) + d[2][2];
+        const T z0 = (d[0][0] + d[1][0]) + d[2][0], z1 = (d[0][1] + d[1][1]) + d[2][1], z2 = (d[0][2] + d[1][2]) + d[2][2];
+        const int n0 = __builtin_popcount(av & 0x49u), n1 = __builtin_popcount(av & (0x49u << 9)), n2 = __builtin_popcount(av & (0x49u << 18));
+        acc += xt[kXY0 + (mask_fold<3>(av, 0) & ly)] * (y1 + y0) - xt[kXY0 + (mask_fold<3>(av, 3) & ry)] * (y1 + y2);
+        acc += xt[kXZ + ((4 * n1 + n0) & lz)] * (z1 + z0) - xt[kXZ + 16 + ((4 * n1 + n2) & rz)] * (z1 + z2);
+    }
+    {  // pairs along y at (x, z)
+        const uint32_t av = m & (m >> 6);
+        T d[3][3];
+#pragma unroll
+        for(int z = 0; z < 3; z++)
+#pragma unroll
+            for(int x = 0; x < 3; x++) d[x][z] = mask_keep(u(x + 9 * z + 6) - u(x + 9 * z), mask_ones(av, x + 9 * z));
+        const T x0 = (d[0][0] + d[0][1]) + d[0][2], x1 = (d[1][0] + d[1][1]) + d[1][2], x2 = (d[2][0] + d[2][1]) + d[2][2];
+        const T z0 = (d[0][0] + d[1][0]) + d[2][0], z1 = (d[0][1] + d[1][1]) + d[2][1], z2 = (d[0][2] + d[1][2]) + d[2][2];
+        const int n0 = __builtin_popcount(av & 7u), n1 = __builtin_popcount(av & (7u << 9)), n2 = __builtin_popcount(av & (7u << 18));
+        acc += xt[kXY1 + (mask_fold<1>(av, 0) & lx)] * (x1 + x0) - xt[kXY1 + (mask_fold<1>(av, 1) & rx)] * (x1 + x2);
+        acc += xt[kYZ + ((4 * n1 + n0) & lz)] * (z1 + z0) - xt[kYZ + 16 + ((4 * n1 + n2) & rz)] * (z1 + z2);
+    }
+    {  // pairs along z at (x, y)
+        const uint32_t av = m & (m >> 18);
+        T d[3][3];
+#pragma unroll
+        for(int y = 0; y < 3; y++)
+#pragma unroll
+            for(int x = 0; x < 3; x++) d[x][y] = mask_keep(u(x + 3 * y + 18) - u(x + 3 * y), mask_ones(av, x + 3 * y));
+        const T x0 = (d[0][0] + d[0][1]) + d[0][2], x1 = (d[1][0] + d[1][1]) + d[1][2], x2 = (d[2][0] + d[2][1]) + d[2][2];
+        const T y0 = (d[0][0] + d[1][0]) + d[2][0], y1 = (d[0][1] + d[1][1]) + d[2][1], y2 = (d[0][2] + d[1][2]) + d[2][2];
+        const int nx0 = __builtin_popcount(av & 0xdbu), nx2 = __builtin_popcount(av & 0x1b6u);   // x in {0,1}, {1,2}
+        const int ny0 = __builtin_popcount(av & 0x3fu), ny2 = __builtin_popcount(av & 0x1f8u);   // y in {0,1}, {1,2}
+        acc += xt[kZX + (nx0 & lx)] * (x1 + x0) - xt[kZX + (nx2 & rx)] * (x1 + x2);
+        acc += xt[kZY + (ny0 & ly)] * (y1 + y0) - xt[kZY + (ny2 & ry)] * (y1 + y2);
+    }
+    return acc;
 }
 
 }  // namespace mono

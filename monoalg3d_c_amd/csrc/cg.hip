@@ -314,14 +314,14 @@ template <typename TV, typename TC, int CM, int PAT, bool FUSE, class Epi>
 __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeom &g, int t, int z0, int z1, const TV *__restrict__ x,
                                              const TV *__restrict__ rz, TV beta, TV *__restrict__ p_out, const Epi &epi,
                                              double (&v)[Epi::NR]) {
-    static_assert(9 * 27 <= kBlock, "one class-row coefficient per thread");
+    static_assert(9 * 27 <= kBlock && kMaskTable == kBlock, "one class-row coefficient or table entry per thread");
     // CM: 0 per-cell rows, 1 class table, 2 code table (7-point rows), 3 rows
     // formed from neighbourhood masks (27-point)
     constexpr bool CLS = CM == 1;
     static_assert(CM != 2 || PAT == 7, "code tables hold 7-point rows");
     static_assert(CM != 3 || PAT == 27, "mask rows are 27-point rows");
     __shared__ TV pl[3 * kPLS];
-    __shared__ TC crows[CLS ? kBlock : 1];  // 9 x 27 class rows, padded to one slot per thread
+    __shared__ TC crows[CLS || CM == 3 ? kBlock : 1];  // 9 x 27 class rows, or the layer's mask table, one slot per thread
     __shared__ TC ctab[CM == 2 ? kCodes * PAT : 1];
     if constexpr(CM == 2) {
         // the code table (identical in every segment: rewriting it is benign);
@@ -385,13 +385,14 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
             pl[slot * kPLS + tid + j * kBlock] = (f.zin && gok[j]) ? val : TV(0);  // lanes past kPL fill padding
         }
     };
-    // class mode: the 9 class rows of a plane (27 slots each) are staged in LDS,
-    // one plane ahead, for tiles on an x or y face and on the boundary planes
+    // mask mode: the weights of a plane's layer are staged in LDS, one plane
+    // ahead; class mode: likewise the 9 class rows of a plane (27 slots each), for tiles on an x or y face and on the boundary planes
     const bool face_xy = CLS && (x0 < g.lo[0] || x0 + kTX - 1 > g.hi[0] || y0 < g.lo[1] || y0 + kTY - 1 > g.hi[1]);
     auto need_rows = [&](int z) { return CLS && (face_xy || z < g.lo[2] || z > g.hi[2]); };
     TC rrow = TC(0);
     auto fetch_rows = [&](int z, bool need) {
         if constexpr(CLS) rrow = op.table[(need && tid < 9 * 27 && need_rows(z)) ? (int64_t)z * 9 * 27 + tid : 0];
+        if constexpr(CM == 3) rrow = op.lt[need ? (int64_t)z * kMaskTable + tid : 0];
     };
     const int tx = tid % kTX, ty = tid / kTX;
     const int gx = x0 + tx;
@@ -451,17 +452,12 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
     auto compute = [&](int z, const Pre(&pre)[kRPT], Pre fpre) {
         const TV *const P3[3] = {pl + ((z + 2) % 3) * kPLS, pl + (z % 3) * kPLS, pl + ((z + 1) % 3) * kPLS};
         TC crow[PAT];
-        // mask rows: the tensors of layers z-1, z, z+1 (clamped at the box
-        // faces, where no neighbour uses them), wave-uniform
-        TC tz[MM ? 3 : 1][6];
+        // mask rows: the layer's normal weights, wave-uniform
+        TC wn[4];
         if constexpr(MM) {
-            const scalar_ptr<TC> lt = as_scalar(op.lt);
+            const scalar_ptr<TC> lt = as_scalar(op.lt + (int64_t)z * kMaskTable + kNormal);
 #pragma unroll
-            for(int l = 0; l < 3; l++) {
-                const int zl = z - 1 + l < 0 ? 0 : (z - 1 + l >= op.nz ? op.nz - 1 : z - 1 + l);
-#pragma unroll
-                for(int k = 0; k < 6; k++) tz[l][k] = lt[zl * 6 + k];
-            }
+            for(int k = 0; k < 4; k++) wn[k] = lt[k];
         }
         bool zf = true;
         if constexpr(CLS) {
@@ -485,14 +481,10 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
             TV acc;
             double dg = 0.0;  // the row's diagonal (Jacobi epilogues only)
             if constexpr(MM) {
-                TC row[27];
-                mask_aniso_row<TC, true>(mk[q], tz, op.geo[0], op.geo[1], op.geo[2], op.geo[3], row);
-                acc = TV(0);
-#pragma unroll
-                for(int k = 0; k < PAT; k++)
-                    acc += (TV)row[slot_of(RowPattern<PAT>::o[k][0], RowPattern<PAT>::o[k][1], RowPattern<PAT>::o[k][2])] *
-                           P3[RowPattern<PAT>::o[k][2] + 1][base + RowPattern<PAT>::o[k][1] * kW + RowPattern<PAT>::o[k][0]];
-                if constexpr(Epi::kDiag) dg = (double)row[13];
+                static_assert(!MM || sizeof(TV) == sizeof(TC), "mask rows are applied in the type of their constants");
+                acc = mask_aniso_apply<TC>(
+                    mk[q], wn, op.alpha, crows,
+                    [&](int k) { return P3[k / 9][base + (k / 3 % 3 - 1) * kW + (k % 3 - 1)]; }, Epi::kDiag ? &dg : nullptr);
             } else if constexpr(PF) {
                 acc = TV(0);
 #pragma unroll
@@ -566,7 +558,7 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
     // there leave the other register set's loads in flight.
     auto half_a = [&](int z) {
         put(ra, (z + 1) % 3);  // plane z+1
-        if constexpr(CLS) crows[tid] = rrow;
+        if constexpr(CLS || MM) crows[tid] = rrow;
         fetch_rows(z + 1, z + 1 < z1);
         fetch(ra, z + 3, z + 3 <= z1);
         __syncthreads();
@@ -580,7 +572,7 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
     for(; z + 1 < z1; z += 2) {
         half_a(z);
         put(rb, (z + 2) % 3);  // plane z+2
-        if constexpr(CLS) crows[tid] = rrow;
+        if constexpr(CLS || MM) crows[tid] = rrow;
         fetch_rows(z + 2, z + 2 < z1);
         fetch(rb, z + 4, z + 4 <= z1);
         __syncthreads();
@@ -1388,7 +1380,7 @@ int CgWorkspace::release() {
 template <typename T> static bool same_view(const OpView<T> &a, const OpView<T> &b) {
     return a.nx == b.nx && a.ny == b.ny && a.nz == b.nz && a.n == b.n && a.pat == b.pat && a.table == b.table &&
            a.table_int == b.table_int && a.percell == b.percell && a.codes == b.codes && a.ctab == b.ctab && a.active == b.active &&
-           a.nbm == b.nbm && a.lt == b.lt && a.geo[0] == b.geo[0] && a.geo[1] == b.geo[1] && a.geo[2] == b.geo[2] && a.geo[3] == b.geo[3];
+           a.nbm == b.nbm && a.lt == b.lt && a.alpha == b.alpha;
 }
 
 static bool same_key(const CgWorkspace::PrefixKey &a, const CgWorkspace::PrefixKey &b) {

@@ -77,20 +77,20 @@ template <typename T> struct OpView {
     const uint8_t *codes;       // code mode: [cell] row code (7-point rows only), else null
     const T *ctab;              // code mode: [code * pat + k], kCodes rows, else null
     const uint8_t *active;      // optional
-    // mask mode (27-point anisotropic rows formed in the kernel, see
-    // aniso_row.h): [cell] neighbourhood mask, [z][6] layer tensors, and
-    // dx, dy, dz, alpha; else null
+    // mask mode (27-point anisotropic rows evaluated from masks, see
+    // aniso_row.h): [cell] neighbourhood mask, [z] layer tables
+    // (mask_layer_table) and the storage term; else null
     const uint32_t *nbm;
     const T *lt;
-    T geo[4];
+    T alpha;
 };
 
 // Mask mode: for 27-point anisotropic rows on per-layer (or uniform) tensors
 // without per-cell conductivity factors, a row is fixed by its layer and which
-// of its 26 neighbours exist and are active.  The FP32 view then carries a
-// 4-byte mask per cell and the inner solver's kernels form each row in FP32
-// registers (aniso_row.h) instead of reading 27 stored coefficients; enabled
-// only after the FP64 form of the same function reproduced every assembled
+// of its 26 neighbours exist and are active.  The solver's views then carry a
+// 4-byte mask per cell and its kernels apply each row as sums of masked
+// differences (aniso_row.h) instead of reading 27 stored coefficients; enabled
+// only after rows formed from the masks in FP64 reproduced every assembled
 // row bit for bit.  MONO_MASK_ROWS=0 keeps the stored FP32 rows.
 //
 // Code mode: when every 7-point row is fixed by which of its six neighbours
@@ -114,8 +114,7 @@ struct Operator {
     uint32_t *nbm = nullptr;
     float *lt32 = nullptr;
     double *lt64 = nullptr;
-    float geo32[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    double geo64[4] = {0.0, 0.0, 0.0, 0.0};
+    double mask_alpha = 0.0;
     uint8_t *codes = nullptr;
     double *ctab64 = nullptr;
     float *ctab32 = nullptr;

@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256) void k_verify_mask_rows(const double *coef27, 
 }
 
 // Try mask mode for the FP32 view; returns 1 when every assembled row matched
-// its mask-formed row (op->nbm, lt32, geo32 set), 0 when not, -1 on error.
+// its mask-formed row (op->nbm, lt32, lt64, mask_alpha set), 0 when not, -1 on error.
 static int try_mask_mode(const AssemblyParams &p, const double *coef27, Operator *op, hipStream_t s) {
     const int64_t n = (int64_t)p.nx * p.ny * p.nz;
     const unsigned grid = (unsigned)((n + 255) / 256);
@@ -594,31 +594,28 @@ static int try_mask_mode(const AssemblyParams &p, const double *coef27, Operator
         (void)hipFree(nbm);
         return 0;
     }
-    // layer tables [nz][6] in FP32 and FP64 (a uniform tensor repeated)
-    std::vector<float> t32((size_t)p.nz * 6);
-    std::vector<double> l64((size_t)p.nz * 6);
-    for(int z = 0; z < p.nz; z++)
-        for(int k = 0; k < 6; k++) {
-            l64[(size_t)z * 6 + k] = t64[(size_t)(lstride ? z : 0) * 6 + k];
-            t32[(size_t)z * 6 + k] = (float)l64[(size_t)z * 6 + k];
+    // layer tables in FP32 and FP64 (a uniform tensor repeated)
+    std::vector<float> t32((size_t)p.nz * kMaskTable);
+    std::vector<double> l64((size_t)p.nz * kMaskTable);
+    for(int z = 0; z < p.nz; z++) {
+        const double *lt[3];
+        for(int l = 0; l < 3; l++) {
+            const int zl = z - 1 + l < 0 ? 0 : (z - 1 + l >= p.nz ? p.nz - 1 : z - 1 + l);
+            lt[l] = &t64[(size_t)(lstride ? zl : 0) * 6];
         }
+        mask_layer_table(lt, p.dx, p.dy, p.dz, &l64[(size_t)z * kMaskTable]);
+    }
+    for(size_t i = 0; i < l64.size(); i++) t32[i] = (float)l64[i];
     if(hipMalloc(&op->lt32, sizeof(float) * t32.size()) != hipSuccess || hipMalloc(&op->lt64, sizeof(double) * l64.size()) != hipSuccess ||
        hipMemcpyAsync(op->lt32, t32.data(), sizeof(float) * t32.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
        hipMemcpyAsync(op->lt64, l64.data(), sizeof(double) * l64.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
        hipStreamSynchronize(s) != hipSuccess) {
         (void)hipFree(nbm);
-        mono_set_error("HIP error uploading the operator's layer tensors");
+        mono_set_error("HIP error uploading the operator's layer tables");
         return -1;
     }
     op->nbm = nbm;
-    op->geo32[0] = (float)p.dx;
-    op->geo32[1] = (float)p.dy;
-    op->geo32[2] = (float)p.dz;
-    op->geo32[3] = (float)p.alpha;
-    op->geo64[0] = p.dx;
-    op->geo64[1] = p.dy;
-    op->geo64[2] = p.dz;
-    op->geo64[3] = p.alpha;
+    op->mask_alpha = p.alpha;
     return 1;
 }
 
@@ -659,7 +656,7 @@ OpView<float> Operator::view32() const {
         OpView<float> v = make_view<float>(*this, nullptr, nullptr, nullptr);
         v.nbm = nbm;
         v.lt = lt32;
-        for(int k = 0; k < 4; k++) v.geo[k] = geo32[k];
+        v.alpha = (float)mask_alpha;
         return v;
     }
     return class_mode ? make_view<float>(*this, table32, tint32, nullptr) : make_view<float>(*this, nullptr, nullptr, percell32);
@@ -669,7 +666,7 @@ OpView<double> Operator::view64_solve() const {
     OpView<double> v = make_view<double>(*this, nullptr, nullptr, nullptr);
     v.nbm = nbm;
     v.lt = lt64;
-    for(int k = 0; k < 4; k++) v.geo[k] = geo64[k];
+    v.alpha = mask_alpha;
     return v;
 }
 
