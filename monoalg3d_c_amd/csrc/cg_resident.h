@@ -50,6 +50,8 @@ struct ResidentPlan {
     ResidentGeom g{};
     unsigned long long *words = nullptr;  // exchanged values of both parities
     unsigned long long *sums = nullptr;   // partial sums of both parities
+    void *cells = nullptr;                // halo cells of every tile
+    int *ncells = nullptr;                // how many each tile has
     uint64_t wait_ticks = 2000000;  // longest wait of a block for another: 20 ms of the 100 MHz clock
     size_t words_bytes = 0;
     size_t sums_bytes = 0;

@@ -24,13 +24,14 @@
 // per iteration carries them and the sums.
 //
 // Measured (one MI355X, whole steps, launches of cg.hip -> here): 300-cell cable
-// TT2006 FP64 133 -> 26 us; 64 x 64 x 16 TT2006 FP64 208 -> 69; 256 x 256
-// Mitchell-Schaeffer FP32+refine, per-cell rows, 173 -> 65; 490k-cell TT2006
-// FP32+refine with holes 321 -> 216; 492k-cell ORd FP32+refine, 27-point rows
-// per cell, 576 -> 482; 4M-cell batch TT2006 FP32+refine 945 -> 769.  What
+// TT2006 FP64 133 -> 25 us; 64 x 64 x 16 TT2006 FP64 208 -> 69; 256 x 256
+// Mitchell-Schaeffer FP32+refine, per-cell rows, 173 -> 54; 490k-cell TT2006
+// FP32+refine with holes 321 -> 178; 492k-cell ORd FP32+refine, 27-point rows
+// per cell, 576 -> 405; 4M-cell batch TT2006 FP32+refine 945 -> 690.  What
 // bounds an iteration: 1.1 us of block sums, divisions and barriers on one
 // block, 3.1 us on 128 blocks (two trips of a word through the memory-side
-// cache), 6-10 us where a block holds 2,000-4,000 cells (LDS reads).
+// cache), 6-14 us where a block holds 2,000-16,000 cells (LDS reads, and the
+// wait for the slowest of the blocks).
 //
 // Exchanges need no grid barrier and no fences.  Every 64-bit word that goes
 // from one block to another carries 32 bits of value and the 32-bit number of
@@ -54,6 +55,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <vector>
 
 #include "cg.h"
 #include "wave_sum.h"
@@ -78,7 +80,20 @@ __device__ __forceinline__ void put_value(u64 *w, uint32_t epoch, double v) {
 }
 
 constexpr int kSums = 3;       // sums of an exchange
-constexpr int kSumWords = 8;   // words of a block's sums (two each, to a whole number of 64 bytes)
+constexpr int kSumWords = 8;   // words of a block's sums: two each, to a line of 64 bytes that only it writes
+constexpr int kSumBlocks = 8;  // blocks whose sums one load of a wave covers
+constexpr int kSumLoads = 16;  // such loads in flight together
+constexpr int kMaxSumWaves = 2;
+
+// One halo cell of a tile.  Listed once per plan: found by every block in every
+// launch (a scan of its tile with divisions, an LDS counter) they took 8 of the
+// 11 us before the first exchange of 490k cells.
+struct HaloCell {
+    uint32_t word;  // index of its value in the word buffer
+    uint32_t cell;  // cell of the box
+    uint32_t ext;   // index in the tile with halo
+    uint32_t pad;
+};
 
 struct ResidentArgs {
     OpView<double> op64;
@@ -92,6 +107,8 @@ struct ResidentArgs {
     const double *tol_dev;
     int max_its, max_outer;
     u64 *words, *sums;
+    const HaloCell *cells;  // [block][halo]
+    const int *ncells;
     u64 wait_ticks;
     ResidentStatus *st;
 };
@@ -102,14 +119,18 @@ struct ResidentArgs {
 struct Shape {
     int threads, rpt;
 };
-constexpr Shape kShapes[] = {{256, 1}, {256, 2}, {512, 4}, {512, 8}, {1024, 1}, {1024, 2}, {1024, 16}};
+constexpr Shape kShapes[] = {{256, 1}, {256, 2}, {512, 2}, {512, 4}, {512, 8}, {512, 32}};
 
 // Whether the rows of own cells are kept in registers for the whole solve
 // (rows stored per cell, where they fit): read again in every iteration they
 // would come from the memory-side cache at a latency that these few waves
 // cannot hide (27-point rows of 492k cells: 40 us an iteration).
 constexpr bool keeps_rows(bool mixed, int P, int T, int rpt, bool table) {
-    return !table && rpt * P * (mixed ? 1 : 2) <= (T == 1024 ? 54 : 64);
+    return !table && rpt * P * (mixed ? 1 : 2) <= (T == 512 ? 112 : 64);
+}
+// Whether own x and b stay in registers through the solve (else read again).
+constexpr bool holds_xb(bool mixed, int P, int rpt, bool table) {
+    return rpt <= 8 && (table ? 0 : rpt * P * (mixed ? 1 : 2)) + 4 * rpt <= 124;
 }
 
 // A domain is solved here whenever its vectors fit (resident_plan) and its rows
@@ -121,9 +142,9 @@ constexpr bool keeps_rows(bool mixed, int P, int T, int rpt, bool table) {
 // Which shapes are built: a table in LDS with few cells per block or many;
 // rows per cell only where they are kept.
 constexpr bool built(bool mixed, int P, int T, int rpt, bool table) {
-    if(rpt == 16) return mixed && table && P == 7;
-    if(table) return T < 1024;
-    return keeps_rows(mixed, P, T, rpt, table) && !(P == 7 && T == 1024);
+    if(rpt == 32) return mixed && table && P == 7;
+    if(T == 512 && rpt == 2) return !table && P != 7;
+    return table || keeps_rows(mixed, P, T, rpt, table);
 }
 
 // table rows of a tile: 9 position classes of each of its layers, or the code rows
@@ -136,14 +157,16 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
 
     const ResidentArgs &a;
     // LDS
-    double *ext64;   // mixed: x with halo (shares its space with ext); else unused
+    double *ext64;   // x with halo (shares its space with ext)
     TV *ext;         // the residual with halo
     TV *hs, *hw;     // halo: s and the received values
+    TV *hp, *hd;     // mixed, halo: p and the correction d
+    double *hx;      // mixed, halo: x
     uint32_t *hword; // halo: index of the value in the word buffer
     uint16_t *hext;  // halo: index in ext
     double *tab64;
     TV *tab;
-    double *part;    // [3][NW] wave sums, then [3] totals
+    double *part;    // [3][NW] wave sums, then [4 kMaxSumWaves][3] sums of blocks'
     int *flags;      // [0] a wait ended without its word, [1] halo count
 
     int tid, lane, wave;
@@ -152,7 +175,8 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     int nh;
     uint32_t meta[RPT];  // ext index | table row << 16
     uint32_t cells[TABLE ? 1 : RPT];  // own cells in the box (rows stored per cell)
-    uint32_t mask;       // bit q: own cell q is in the box; bit 16 + q: a neighbour tile needs it
+    uint32_t mask;       // bit q: own cell q is in the box
+    uint32_t edge;       // bit q: a neighbour tile needs it
     uint32_t epoch;
     TV w[RPT];
 
@@ -172,12 +196,8 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         lz = a.by == 1 ? r : (int)__umulhi((uint32_t)r, a.div_by);
         ly = r - lz * a.by;
     }
-    __device__ __forceinline__ int64_t ext_cell(int e) const {
-        const int exx = e % ex, r = e / ex, eyy = r % ey, ezz = r / ey;
-        return (x0 + exx - hx_) + (int64_t)a.op64.nx * ((y0 + eyy - hy_) + (int64_t)a.op64.ny * (z0 + ezz - hz_));
-    }
-
-    __device__ __forceinline__ void setup(char *lds) {
+    // this thread's place: own cells and their masks
+    __device__ __forceinline__ void place() {
         tid = threadIdx.x;
         lane = tid & 63;
         wave = tid >> 6;
@@ -186,6 +206,25 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         x0 = btx * a.bx;
         y0 = bty * a.by;
         z0 = btz * a.bz;
+        mask = edge = 0;
+        const int tile = a.bx * a.by * a.bz;
+#pragma unroll
+        for(int q = 0; q < RPT; q++) {
+            const int l = local(q);
+            int lx, ly, lz;
+            split(l, lx, ly, lz);
+            const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
+            if(l < tile && gx < nx && gy < ny && gz < nz) {
+                mask |= 1u << q;
+                if((lx == 0 && gx > 0) || (lx == a.bx - 1 && gx < nx - 1) || (ly == 0 && gy > 0) || (ly == a.by - 1 && gy < ny - 1) ||
+                   (lz == 0 && gz > 0) || (lz == a.bz - 1 && gz < nz - 1))
+                    edge |= 1u << q;
+            }
+        }
+    }
+
+    __device__ __forceinline__ void setup(char *lds) {
+        const int nx = a.op64.nx, ny = a.op64.ny, nz = a.op64.nz;
         hx_ = nx > 1;
         hy_ = ny > 1;
         hz_ = nz > 1;
@@ -205,9 +244,14 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         ext = (TV *)ext64;
         hs = (TV *)take(sizeof(TV) * a.halo);
         hw = (TV *)take(sizeof(TV) * a.halo);
+        if constexpr(MIXED) {
+            hp = (TV *)take(sizeof(TV) * a.halo);
+            hd = (TV *)take(sizeof(TV) * a.halo);
+            hx = (double *)take(sizeof(double) * a.halo);
+        }
         hword = (uint32_t *)take(sizeof(uint32_t) * a.halo);
         hext = (uint16_t *)take(sizeof(uint16_t) * a.halo);
-        part = (double *)take(sizeof(double) * (3 * NW + 3));
+        part = (double *)take(sizeof(double) * kSums * (NW + 4 * kMaxSumWaves));
         flags = (int *)take(2 * sizeof(int));
         if constexpr(TABLE) {
             const int rows = a.op64.codes ? kCodes : 9 * a.bz;
@@ -216,70 +260,42 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             fill_table(a.op64, rows, MIXED ? tab64 : (double *)tab);
             if constexpr(MIXED) fill_table(a.op32, rows, (float *)tab);
         }
-        if(tid == 0) {
-            flags[0] = __hip_atomic_load(&a.st->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kResidentGoing;
-            flags[1] = 0;
+        if(tid == 0) flags[0] = __hip_atomic_load(&a.st->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kResidentGoing;
+        nh = a.nblocks > 1 ? a.ncells[blockIdx.x] : 0;
+        for(int i = tid; i < nh; i += T) {
+            const HaloCell h = a.cells[(size_t)blockIdx.x * a.halo + i];
+            hword[i] = h.word;
+            hext[i] = (uint16_t)h.ext;
         }
-        __syncthreads();
-        // own cells
-        mask = 0;
-        const int tile = a.bx * a.by * a.bz;
 #pragma unroll
         for(int q = 0; q < RPT; q++) {
-            const int l = local(q);
             int lx, ly, lz;
-            split(l, lx, ly, lz);
+            split(local(q), lx, ly, lz);
             const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
             meta[q] = 0;
             if constexpr(!TABLE) cells[q] = 0;
-            if(l < tile && gx < nx && gy < ny && gz < nz) {
-                mask |= 1u << q;
-                if((lx == 0 && gx > 0) || (lx == a.bx - 1 && gx < nx - 1) || (ly == 0 && gy > 0) || (ly == a.by - 1 && gy < ny - 1) ||
-                   (lz == 0 && gz > 0) || (lz == a.bz - 1 && gz < nz - 1))
-                    mask |= 1u << (16 + q);
+            if(own(q)) {
+                const uint32_t c = (uint32_t)(gx + (int64_t)nx * (gy + (int64_t)ny * gz));
                 uint32_t row = 0;
-                if constexpr(TABLE) {
-                    if(a.op64.codes) row = a.op64.codes[gx + (int64_t)nx * (gy + (int64_t)ny * gz)];
-                    else row = (lz * 3 + pos(gy, ny)) * 3 + pos(gx, nx);
-                }
-                if constexpr(!TABLE) cells[q] = (uint32_t)(gx + (int64_t)nx * (gy + (int64_t)ny * gz));
+                if constexpr(TABLE) row = a.op64.codes ? a.op64.codes[c] : (lz * 3 + pos(gy, ny)) * 3 + pos(gx, nx);
+                if constexpr(!TABLE) cells[q] = c;
                 meta[q] = (uint32_t)((lx + hx_) + ex * ((ly + hy_) + ey * (lz + hz_))) | (row << 16);
             }
         }
-        // halo cells: those of the box that lie next to the tile and that the
-        // row pattern reaches.  Their order in the list is arbitrary; nothing is
-        // summed over them.
-        for(int e = tid; e < ne; e += T) {
-            const int lx = e % ex - hx_, r = e / ex, ly = r % ey - hy_, lz = r / ey - hz_;
-            const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
-            const int out = (lx < 0 || lx >= a.bx) + (ly < 0 || ly >= a.by) + (lz < 0 || lz >= a.bz);
-            if(out == 0 || (P == 7 && out > 1)) continue;
-            if(gx < 0 || gx >= nx || gy < 0 || gy >= ny || gz < 0 || gz >= nz) continue;
-            const int i = atomicAdd(&flags[1], 1);
-            const int ox = gx / a.bx, oy = gy / a.by, oz = gz / a.bz;
-            const int l = (gx - ox * a.bx) + a.bx * ((gy - oy * a.by) + a.by * (gz - oz * a.bz));
-            hext[i] = (uint16_t)e;
-            hword[i] = (uint32_t)((ox + a.tx * (oy + a.ty * oz)) * (RPT * T) + l);
-        }
         __syncthreads();
-        nh = flags[1];
     }
 
     static __device__ __forceinline__ int pos(int i, int len) { return i == 0 ? 0 : (i == len - 1 ? 2 : 1); }
 
     // rows [row][P] of the tile: the classes of its layers, or the codes
     template <typename TC> __device__ __forceinline__ void fill_table(const OpView<TC> &op, int rows, TC *t) {
-        for(int i = tid; i < rows; i += T) {
-            const TC *src;
-            bool in = true;
-            if(op.codes) src = op.ctab + i * P;
+        for(int j = tid; j < rows * P; j += T) {
+            const int i = j / P, k = j - i * P;
+            if(op.codes) t[j] = op.ctab[j];
             else {
-                in = z0 + i / 9 < op.nz;
-                src = op.table + (in ? ((int64_t)z0 * 9 + i) * 27 : 0);
+                const bool in = z0 + i / 9 < op.nz;
+                t[j] = op.table[(in ? ((int64_t)z0 * 9 + i) * 27 : 0) + slot_of(RowPattern<P>::o[k][0], RowPattern<P>::o[k][1], RowPattern<P>::o[k][2])];
             }
-#pragma unroll
-            for(int k = 0; k < P; k++)
-                t[i * P + k] = op.codes ? src[k] : src[slot_of(RowPattern<P>::o[k][0], RowPattern<P>::o[k][1], RowPattern<P>::o[k][2])];
         }
     }
 
@@ -335,10 +351,10 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             for(int k = 0; k < P; k++) {
                 acc += *row * v[e + d.of(k)];
                 row += n;
-                breathe<T == 1024>(k);
             }
         }
-        if constexpr(RPT > 1) __builtin_amdgcn_sched_barrier(0);  // one row's operands in registers at a time
+        // one row's operands in registers at a time, two rows' with a table
+        if(RPT > 1 && (!TABLE || q % 2 == 1)) __builtin_amdgcn_sched_barrier(0);
         return acc;
     }
 
@@ -367,6 +383,60 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         for(int k = 0; k < N; k++) h[k] = (uint32_t)v[k];
     }
 
+    // waves that add up the blocks' sums; the others receive the halo
+    __device__ __forceinline__ int sum_waves() const { return a.nblocks > kSumBlocks * kSumLoads ? kMaxSumWaves : 1; }
+
+    // the neighbour eight lanes on, round each row of 16
+    static __device__ __forceinline__ double row_ror8(double v) {
+        struct Halves {
+            int lo, hi;
+        } h = __builtin_bit_cast(Halves, v);
+        h.lo = __builtin_amdgcn_update_dpp(0, h.lo, 0x128, 0xf, 0xf, false);
+        h.hi = __builtin_amdgcn_update_dpp(0, h.hi, 0x128, 0xf, 0xf, false);
+        return __builtin_bit_cast(double, h);
+    }
+
+    // Adds a value of blocks i + sub, i + sub + 8, ... (N of them) to sum; valid
+    // in the lanes of low words.
+    template <int N>
+    __device__ __forceinline__ void add_sums(const u64 *S, int i, int sub, int word, double &sum, bool &bad) {
+        const u64 *p[N];
+#pragma unroll
+        for(int j = 0; j < N; j++) {
+            const int b = i + sub + j * kSumBlocks;
+            p[j] = S + (size_t)kSumWords * (b < a.nblocks ? b : a.nblocks - 1) + word;
+        }
+        uint32_t h[N];
+        await<N>(p, h, bad);
+#pragma unroll
+        for(int j = 0; j < N; j++) {
+            const uint32_t high = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h[j], 0xB1, 0xf, 0xf, false);  // the other lane of the pair
+            if(i + sub + j * kSumBlocks < a.nblocks) sum += join(h[j], high);
+        }
+    }
+
+    // Halo values i0, i0 + step, ... (M of them; past the end: the first again).
+    template <typename T2, int M, class Store>
+    __device__ __forceinline__ void receive(const u64 *W, int i0, int step, bool &bad, Store &&store) {
+        constexpr int K = kWords<T2>;
+        const u64 *p[M * K];
+        int i[M];
+#pragma unroll
+        for(int j = 0; j < M; j++) {
+            i[j] = i0 + j * step < nh ? i0 + j * step : i0;
+            const u64 *w = W + (size_t)K * hword[i[j]];
+#pragma unroll
+            for(int k = 0; k < K; k++) p[j * K + k] = w + k;
+        }
+        uint32_t h[M * K];
+        await<M * K>(p, h, bad);
+#pragma unroll
+        for(int j = 0; j < M; j++) {
+            if constexpr(K == 1) store(i[j], __uint_as_float(h[j]));
+            else store(i[j], join(h[2 * j], h[2 * j + 1]));
+        }
+    }
+
     // Wait for all blocks' sums (wave 0) and the halo values (the other waves)
     // of this exchange; both totals to every thread.  False when a wait ended
     // without its words.
@@ -374,50 +444,47 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         const u64 *W = a.words + (size_t)(epoch & 1) * ((size_t)a.nblocks * RPT * T * 2);
         const u64 *S = a.sums + (size_t)(epoch & 1) * ((size_t)a.nblocks * kSumWords);
         bool bad = false;
-        if(wave == 0) {
-            double sum[kSums] = {0.0, 0.0, 0.0};
-            for(int i = lane; i < a.nblocks; i += 128) {
-                const bool two = i + 64 < a.nblocks;
-                const u64 *q0 = &S[kSumWords * i], *q1 = &S[kSumWords * (two ? i + 64 : i)];
-                const u64 *const p[12] = {q0, q0 + 1, q0 + 2, q0 + 3, q0 + 4, q0 + 5, q1, q1 + 1, q1 + 2, q1 + 3, q1 + 4, q1 + 5};
-                uint32_t h[12];
-                await<12>(p, h, bad);
-#pragma unroll
-                for(int k = 0; k < kSums; k++) {
-                    sum[k] += join(h[2 * k], h[2 * k + 1]);
-                    if(two) sum[k] += join(h[6 + 2 * k], h[7 + 2 * k]);
-                }
+        const int nsum = sum_waves();
+        if(wave < nsum) {
+            // lane 8 i + k takes word k of block i of eight: a load touches
+            // eight lines once, where a lane to a block touched 64 lines in
+            // each of six loads (168 blocks: an exchange 5.9 -> 4.9 us).  Each
+            // line stays one block's: with the sums laid out by word, eight
+            // blocks to a line, 128 blocks took 2.8 us where now it is 2.3.
+            const int word = (lane & 7) < 2 * kSums ? lane & 7 : 0, sub = lane >> 3;
+            double sum = 0.0;
+            for(int i = wave * kSumBlocks * kSumLoads; i < a.nblocks; i += nsum * kSumBlocks * kSumLoads) {
+                const int left = (a.nblocks - i + kSumBlocks - 1) / kSumBlocks;
+                if(left <= kSumLoads / 4) add_sums<kSumLoads / 4>(S, i, sub, word, sum, bad);
+                else if(left <= kSumLoads / 2) add_sums<kSumLoads / 2>(S, i, sub, word, sum, bad);
+                else add_sums<kSumLoads>(S, i, sub, word, sum, bad);
             }
-            wave_sums(sum);
-            if(lane == kSumLane) {
-#pragma unroll
-                for(int k = 0; k < kSums; k++) part[kSums * NW + k] = sum[k];
-            }
+            sum += row_ror8(sum);
+            // four rows of 16 lanes: their sums are added after the barrier
+            if((lane & 15) < 2 * kSums && (lane & 1) == 0) part[kSums * NW + (wave * 4 + (lane >> 4)) * kSums + ((lane & 15) >> 1)] = sum;
         } else {
-            constexpr int M = sizeof(T2) == 4 ? 4 : 2;  // values waited for together
-            for(int i0 = tid - 64; i0 < nh; i0 += M * (T - 64)) {
-                const u64 *p[4];
-                int i[M];
-#pragma unroll
-                for(int j = 0; j < M; j++) {
-                    i[j] = i0 + j * (T - 64) < nh ? i0 + j * (T - 64) : i0;
-                    const u64 *w = W + (size_t)kWords<T2> * hword[i[j]];
-                    p[j * kWords<T2>] = w;
-                    if constexpr(sizeof(T2) == 8) p[2 * j + 1] = w + 1;
-                }
-                uint32_t h[4];
-                await<4>(p, h, bad);
-#pragma unroll
-                for(int j = 0; j < M; j++) {
-                    if constexpr(sizeof(T2) == 4) store(i[j], __uint_as_float(h[j]));
-                    else store(i[j], join(h[2 * j], h[2 * j + 1]));
-                }
+            // (the edge cells' words keep their places in the tile, each cell
+            // written by its own thread as soon as it is known: packed face by
+            // face, in fewer lines but several waves to a line, the exchange of
+            // 128 blocks took 0.5 us longer.)
+            // The values of up to four words a lane are waited for together,
+            // no more than this wave has left
+            const int step = T - 64 * nsum;
+            for(int i0 = tid - 64 * nsum; i0 < nh; ) {
+                const int left = __builtin_amdgcn_readfirstlane((nh - (i0 - lane) + step - 1) / step);
+                if(left == 1) receive<T2, 1>(W, i0, step, bad, store), i0 += step;
+                else if(left == 2 || sizeof(T2) == 8) receive<T2, 2>(W, i0, step, bad, store), i0 += 2 * step;
+                else receive<T2, sizeof(T2) == 8 ? 2 : 4>(W, i0, step, bad, store), i0 += 4 * step;
             }
         }
         if(bad) flags[0] = 1;
         __syncthreads();
 #pragma unroll
-        for(int k = 0; k < kSums; k++) t[k] = part[kSums * NW + k];
+        for(int k = 0; k < kSums; k++) {
+            const double *v = part + kSums * NW + k;
+            t[k] = (v[0] + v[kSums]) + (v[2 * kSums] + v[3 * kSums]);
+            if(nsum == 2) t[k] += (v[4 * kSums] + v[5 * kSums]) + (v[6 * kSums] + v[7 * kSums]);
+        }
         return flags[0] == 0;
     }
 
@@ -431,10 +498,9 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         u64 *W = a.words + (size_t)(epoch & 1) * ((size_t)a.nblocks * RPT * T * 2);
         u64 *S = a.sums + (size_t)(epoch & 1) * ((size_t)a.nblocks * kSumWords);
 #pragma unroll
-        for(int q = 0; q < RPT; q++)
-        {
-            if((mask >> (16 + q)) & 1u) put_value(W + (size_t)kWords<T2> * ((size_t)blockIdx.x * (RPT * T) + local(q)), epoch, value(q));
-            breathe<RPT == 16, 4>(q);
+        for(int q = 0; q < RPT; q++) {
+            if((edge >> q) & 1u) put_value(W + (size_t)kWords<T2> * ((size_t)blockIdx.x * (RPT * T) + local(q)), epoch, value(q));
+            breathe<RPT == 32, 8>(q);
         }
         wave_sums(t);
         if(lane == kSumLane) {
@@ -465,9 +531,20 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     // zero), rr = r.r.  Returns the status through its arguments; false after a
     // wait that did not end.
     __device__ __forceinline__ bool cg(TV (&d)[RPT], double rr, double tol, int &iters, double &rr_end) {
-        TV p[RPT], s[RPT];
+        // With many cells a thread p lies in LDS, where x was: in registers the
+        // 32 cells of a thread spilled (4M-cell batch: 950 -> 720 us a step).
+        constexpr bool kLdsP = MIXED && RPT == 32;
+        TV preg[kLdsP ? 1 : RPT], s[RPT];
+        TV *const pl = ext + ex * ey * ez;
+        auto p = [&](int q) -> TV & {
+            if constexpr(kLdsP) return pl[at(q)];
+            else return preg[q];
+        };
 #pragma unroll
-        for(int q = 0; q < RPT; q++) p[q] = s[q] = TV(0);
+        for(int q = 0; q < RPT; q++) {
+            s[q] = TV(0);
+            if(!kLdsP || own(q)) p(q) = TV(0);
+        }
         TV keep[kKeepRows ? RPT : 1][kKeepRows ? P : 1];
         if constexpr(kKeepRows) {
 #pragma unroll
@@ -478,7 +555,10 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                 for(int k = 0; k < P; k++) keep[q][k] = (view()->percell + (int64_t)k * view()->n)[c];
             }
         }
-        for(int i = tid; i < nh; i += T) hs[i] = TV(0);
+        for(int i = tid; i < nh; i += T) {
+            hs[i] = TV(0);
+            if constexpr(MIXED) hp[i] = hd[i] = TV(0);
+        }
         __syncthreads();
         double beta = 0.0, pq = 0.0;
         for(int k = 0;; k++) {
@@ -494,7 +574,6 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
 #pragma unroll
                     for(int j = 0; j < P; j++) {
                         w[q] += keep[q][j] * ext[e + sd.of(j)];
-                        breathe<T == 1024>(j);
                     }
                 } else {
                     w[q] = row_times<TV>(*view(), tab, q, ext);
@@ -502,7 +581,7 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                 const TV r = ext[at(q)];
                 t[0] += (double)r * (double)r;
                 t[1] += (double)r * (double)w[q];
-                t[2] += (double)r * (double)s[q] + (double)p[q] * (double)w[q];
+                t[2] += (double)r * (double)s[q] + (double)p(q) * (double)w[q];
             }
             if(!exchange<TV>([&](int q) { return w[q]; }, t, [&](int i, TV v) { hw[i] = v; })) return false;
             if(k > 0) {
@@ -519,20 +598,32 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                 if(!own(q)) continue;
                 TV &r = ext[at(q)];
                 const TV ro = r;
-                s[q] = w[q] + be * s[q];
-                p[q] = ro + be * p[q];
-                d[q] = d[q] + al * p[q];
-                r = ro - al * s[q];
-                breathe<RPT == 16, 4>(q);
+                s[q] = fused(be, s[q], w[q]);
+                const TV pv = fused(be, p(q), ro);
+                p(q) = pv;
+                d[q] = fused(al, pv, d[q]);
+                r = fused(-al, s[q], ro);
+                breathe<RPT == 32, 8>(q);
             }
             for(int i = tid; i < nh; i += T) {
-                const TV sv = hw[i] + be * hs[i];
+                TV &r = ext[hext[i]];
+                const TV ro = r, sv = fused(be, hs[i], hw[i]);
                 hs[i] = sv;
-                ext[hext[i]] -= al * sv;
+                if constexpr(MIXED) {
+                    const TV pv = fused(be, hp[i], ro);
+                    hp[i] = pv;
+                    hd[i] = fused(al, pv, hd[i]);
+                }
+                r = fused(-al, sv, ro);
             }
             __syncthreads();
         }
     }
+
+    // The halo repeats its owners' operations, so that its r, p, d and x are
+    // theirs bit for bit: fused on both sides by name, not as the compiler likes.
+    static __device__ __forceinline__ float fused(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
+    static __device__ __forceinline__ double fused(double x, double y, double z) { return __builtin_fma(x, y, z); }
 
     __device__ __forceinline__ const OpView<TV> *view() const {
         if constexpr(MIXED) return &a.op32;
@@ -564,6 +655,17 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     }
 
     __device__ __forceinline__ void run(char *lds) {
+        place();
+        constexpr bool kHold = holds_xb(MIXED, P, RPT, TABLE);
+        double xh[kHold ? RPT : 1], bh[kHold ? RPT : 1];
+        if constexpr(kHold) {
+#pragma unroll
+            for(int q = 0; q < RPT; q++) {
+                const int64_t c = own(q) ? cell(q) : 0;
+                xh[q] = a.x[c];
+                bh[q] = a.b[c];
+            }
+        }
         setup(lds);
         if(flags[0]) return;  // an earlier solve, or another block of this one, has stopped the run
         epoch = a.st->epoch;
@@ -572,29 +674,36 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         double tol_abs = 0.0, rr = 0.0;
         int inner_total = 0, corrections = 0;
         for(int sweep = 0;; sweep++) {
-            // x with its halo into LDS
+            // x with its halo into LDS, corrected by the last sweep's d
             zero_ext(2 * ne);
-            if(sweep == 0) {
 #pragma unroll
-                for(int q = 0; q < RPT; q++)
-                    if(own(q)) ext64[at(q)] = a.x[cell(q)];
-                for(int i = tid; i < nh; i += T) ext64[hext[i]] = a.x[ext_cell(hext[i])];
-            } else {
-                // corrected by the last sweep's d
-                double none[kSums] = {0.0, 0.0, 0.0};
-#pragma unroll
-                for(int q = 0; q < RPT; q++) {
-                    if(!own(q)) continue;
+            for(int q = 0; q < RPT; q++) {
+                if(!own(q)) continue;
+                double xn;
+                if constexpr(kHold) {
+                    if(sweep > 0) xh[q] += (double)d[q];
+                    xn = xh[q];
+                } else {
                     const int64_t c = cell(q);
-                    const double xn = a.x[c] + (double)d[q];
-                    a.x[c] = xn;
-                    ext64[at(q)] = xn;
-                    breathe<RPT == 16, 4>(q);
+                    xn = a.x[c];
+                    if(sweep > 0) {
+                        xn += (double)d[q];
+                        a.x[c] = xn;
+                    }
                 }
-                if(!exchange<double>([&](int q) { return ext64[at(q)]; }, none, [&](int i, double v) { ext64[hext[i]] = v; })) {
-                    timed_out();
-                    return;
+                ext64[at(q)] = xn;
+                breathe<RPT == 32, 8>(q);
+            }
+            for(int i = tid; i < nh; i += T) {
+                double xn;
+                if constexpr(MIXED) {
+                    if(sweep == 0) xn = a.x[a.cells[(size_t)blockIdx.x * a.halo + i].cell];
+                    else xn = hx[i] + (double)hd[i];
+                    hx[i] = xn;
+                } else {
+                    xn = a.x[a.cells[(size_t)blockIdx.x * a.halo + i].cell];
                 }
+                ext64[hext[i]] = xn;
             }
             __syncthreads();
             // r = b - A x in FP64, r.r, b.b
@@ -604,12 +713,14 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             for(int q = 0; q < RPT; q++) {
                 r[q] = TV(0);
                 if(!own(q)) continue;
-                const double bc = a.b[cell(q)];
+                double bc;
+                if constexpr(kHold) bc = bh[q];
+                else bc = a.b[cell(q)];
                 const double rc = bc - row_times<double>(a.op64, MIXED ? tab64 : (const double *)tab, q, ext64);
                 r[q] = (TV)rc;
                 t[0] += rc * rc;
                 t[1] += bc * bc;
-                breathe<RPT == 16, 2>(q);
+                breathe<RPT == 32, 4>(q);
             }
             __syncthreads();
             zero_ext(MIXED ? ne : 2 * ne);
@@ -631,7 +742,10 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                     return;
                 }
 #pragma unroll
-                for(int q = 0; q < RPT; q++) d[q] = own(q) ? a.x[cell(q)] : 0.0;
+                for(int q = 0; q < RPT; q++) {
+                    if constexpr(kHold) d[q] = xh[q];
+                    else d[q] = own(q) ? a.x[cell(q)] : 0.0;
+                }
                 if(!cg(d, rr, tol_abs, iters, rr_end)) {
                     timed_out();
                     return;
@@ -643,6 +757,13 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
                 return;
             } else {
                 if(!(rr > tol_abs) || sweep >= a.max_outer || rr != rr) {
+                    if constexpr(kHold) {
+                        if(sweep > 0) {
+#pragma unroll
+                            for(int q = 0; q < RPT; q++)
+                                if(own(q)) a.x[cell(q)] = xh[q];
+                        }
+                    }
                     note(inner_total + 1, corrections + 1, inner_total, rr);
                     return;
                 }
@@ -692,11 +813,10 @@ template <bool MIXED, class F> void with_kernel(int P, int threads, int rpt, boo
         };
         one(IC<256>{}, IC<1>{});
         one(IC<256>{}, IC<2>{});
+        one(IC<512>{}, IC<2>{});
         one(IC<512>{}, IC<4>{});
         one(IC<512>{}, IC<8>{});
-        one(IC<1024>{}, IC<1>{});
-        one(IC<1024>{}, IC<2>{});
-        one(IC<1024>{}, IC<16>{});
+        one(IC<512>{}, IC<32>{});
     };
     auto by_table = [&](auto P_) {
         if(table) by_shape(P_, IC<1>{});
@@ -717,7 +837,7 @@ template <typename TC> int storage(const OpView<TC> &op) {
 size_t lds_bytes(bool mixed, int P, const ResidentGeom &g, int mode, const int (&h)[3]) {
     auto up = [](size_t b) { return (b + 15) / 16 * 16; };
     const size_t ne = (size_t)(g.bx + 2 * h[0]) * (g.by + 2 * h[1]) * (g.bz + 2 * h[2]), w = mixed ? 4 : 8, nh = (size_t)g.halo;
-    size_t b = up(8 * ne) + 2 * up(w * nh) + up(4 * nh) + up(2 * nh) + up(8 * (3 * (g.threads / 64) + 3)) + up(8);
+    size_t b = up(8 * ne) + 2 * up(w * nh) + (mixed ? 2 * up(w * nh) + up(8 * nh) : 0) + up(4 * nh) + up(2 * nh) + up(8 * kSums * (g.threads / 64 + 4 * kMaxSumWaves)) + up(8);
     if(mode > 0) {
         const size_t rows = mode == 2 ? kCodes : 9 * (size_t)g.bz;
         b += up(w * rows * P) + (mixed ? up(8 * rows * P) : 0);
@@ -758,10 +878,13 @@ bool best_tiles(const int (&L)[3], int P, bool mixed, int mode, Shape shape, int
                 g.lds = lds_bytes(mixed, P, g, mode, h);
                 if(g.lds > 160 * 1024) continue;
                 const int blocks = tx * ty * tz;
-                // us: block sums, the sums of all blocks, halo words and rows per thread
-                const double c = 1.0 + (T > 256 ? 0.3 : 0.0) + (T > 512 ? 0.5 : 0.0) + (blocks > 1 ? 0.8 + 0.006 * blocks : 0.0) +
+                // us: block sums, the sums of all blocks, halo words and rows per
+                // thread (128 -> 256 blocks with half the rows: 64 x 64 x 16 FP64
+                // 69 -> 75 us a step, 256 x 256 FP32 53 -> 59; 168 blocks of 2,900
+                // cells -> 252 of 1,900: 200 -> 179)
+                const double c = 1.0 + (T > 256 ? 0.3 : 0.0) + (blocks > 1 ? 0.8 + 0.006 * blocks : 0.0) +
                                  0.08 * ((g.halo + T - 65) / (T - 64)) * (mixed ? 1.0 : 1.5) +
-                                 ((cells + T - 1) / T) * (T / 256) * (0.03 + 0.012 * P) * (mixed ? 1.0 : 1.5);
+                                 ((cells + T - 1) / T) * (T / 256) * (0.05 + 0.03 * P);
                 if(!found || c < *cost) {
                     found = true;
                     *best = g;
@@ -771,6 +894,49 @@ bool best_tiles(const int (&L)[3], int P, bool mixed, int mode, Shape shape, int
         }
     }
     return found;
+}
+
+// Halo cells of every tile: those of the box that lie next to it and that the
+// row pattern reaches, [block][g.halo], and their counts.  Direction by
+// direction, so that consecutive cells are consecutive words of one owner.
+std::vector<HaloCell> halo_cells(const int (&L)[3], int P, const ResidentGeom &g, std::vector<int> *count) {
+    const int blocks = g.tx * g.ty * g.tz, b[3] = {g.bx, g.by, g.bz}, t[3] = {g.tx, g.ty, g.tz};
+    const int h[3] = {L[0] > 1, L[1] > 1, L[2] > 1};
+    std::vector<HaloCell> list((size_t)blocks * g.halo);
+    count->assign(blocks, 0);
+    for(int blk = 0; blk < blocks; blk++) {
+        const int tile[3] = {blk % t[0], (blk / t[0]) % t[1], blk / (t[0] * t[1])};
+        int n = 0;
+        for(int dir = 0; dir < 27; dir++) {
+            const int o[3] = {dir % 3 - 1, dir / 3 % 3 - 1, dir / 9 - 1};
+            const int out = abs(o[0]) + abs(o[1]) + abs(o[2]);
+            if(out == 0 || (P == 7 && out > 1)) continue;
+            int lo[3], hi[3], owner[3];
+            bool in = true;
+            for(int k = 0; k < 3; k++) {
+                owner[k] = tile[k] + o[k];
+                in = in && owner[k] >= 0 && owner[k] < t[k];
+                const int len = std::min(b[k], L[k] - tile[k] * b[k]);  // the tile's cells in the box
+                lo[k] = o[k] < 0 ? -1 : (o[k] > 0 ? b[k] : 0);
+                hi[k] = o[k] == 0 ? len - 1 : lo[k];
+            }
+            if(!in) continue;
+            const uint32_t first = (uint32_t)((owner[0] + t[0] * (owner[1] + t[1] * owner[2])) * (g.rpt * g.threads));
+            for(int z = lo[2]; z <= hi[2]; z++)
+                for(int y = lo[1]; y <= hi[1]; y++)
+                    for(int x = lo[0]; x <= hi[0]; x++) {
+                        const int l[3] = {x - o[0] * b[0], y - o[1] * b[1], z - o[2] * b[2]};  // its place in the owner
+                        HaloCell &c = list[(size_t)blk * g.halo + n++];
+                        c.word = first + (uint32_t)(l[0] + b[0] * (l[1] + b[1] * l[2]));
+                        c.cell = (uint32_t)((tile[0] * b[0] + x) +
+                                            (int64_t)L[0] * ((tile[1] * b[1] + y) + (int64_t)L[1] * (tile[2] * b[2] + z)));
+                        c.ext = (uint32_t)((x + h[0]) + (b[0] + 2 * h[0]) * ((y + h[1]) + (b[1] + 2 * h[1]) * (z + h[2])));
+                        c.pad = 0;
+                    }
+        }
+        (*count)[blk] = n;
+    }
+    return list;
 }
 
 }  // namespace
@@ -829,6 +995,12 @@ int resident_plan(ResidentPlan *p, const OpView<double> &op64, const OpView<floa
         p->sums_bytes = sizeof(u64) * 2 * (size_t)blocks * kSumWords;
         MONO_CHECK(hipMalloc(&p->words, p->words_bytes));
         MONO_CHECK(hipMalloc(&p->sums, p->sums_bytes));
+        std::vector<int> count;
+        const std::vector<HaloCell> list = halo_cells(L, P, g, &count);
+        MONO_CHECK(hipMalloc(&p->cells, sizeof(HaloCell) * list.size()));
+        MONO_CHECK(hipMalloc(&p->ncells, sizeof(int) * count.size()));
+        MONO_CHECK(hipMemcpy(p->cells, list.data(), sizeof(HaloCell) * list.size(), hipMemcpyHostToDevice));
+        MONO_CHECK(hipMemcpy(p->ncells, count.data(), sizeof(int) * count.size(), hipMemcpyHostToDevice));
     }
     if(getenv("MONO_TRACE_SLOTS"))
         fprintf(stderr, "[mono] resident solve %s, mode %d, %d-point rows, %dx%dx%d: %dx%dx%d tiles of %dx%dx%d, %d threads, %d cells per thread, %zu bytes of LDS, %d per CU%s\n",
@@ -841,6 +1013,8 @@ int resident_plan(ResidentPlan *p, const OpView<double> &op64, const OpView<floa
 int resident_release(ResidentPlan *p) {
     if(p->words) MONO_CHECK(hipFree(p->words));
     if(p->sums) MONO_CHECK(hipFree(p->sums));
+    if(p->cells) MONO_CHECK(hipFree(p->cells));
+    if(p->ncells) MONO_CHECK(hipFree(p->ncells));
     *p = ResidentPlan();
     return 0;
 }
@@ -881,6 +1055,8 @@ int resident_launch(const ResidentPlan &p, const OpView<double> &op64, const OpV
     a.max_outer = cfg.max_outer;
     a.words = p.words;
     a.sums = p.sums;
+    a.cells = (const HaloCell *)p.cells;
+    a.ncells = p.ncells;
     a.wait_ticks = p.wait_ticks;
     a.st = st;
     hipError_t err = hipSuccess;

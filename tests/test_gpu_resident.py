@@ -51,8 +51,8 @@ def _run(shape, resident, kind, precision, steps, **env):
 
 
 # one block and many; tiles that fill their block and tiles cut by the box's
-# end; axes of one, two and three cells; 256, 512 and 1024 threads and 1, 2, 4,
-# 8 and 16 cells per thread (the largest three only with few steps)
+# end; axes of one, two and three cells; 256 and 512 threads and 1, 2, 4, 8 and
+# 32 cells per thread (the largest three only with few steps)
 SHAPES = {
     "plain": [(300, 1, 1), (1, 700, 1), (1, 1, 65), (2, 2, 2), (40, 1, 7), (33, 17, 9), (64, 64, 1), (100, 80, 20)],
     "holes": [(20, 14, 4), (257, 3, 1), (129, 67, 1), (1100, 1000, 1), (1700, 1500, 1), (120, 100, 33)],
