@@ -26,8 +26,8 @@
 // Measured (one MI355X, whole steps, launches of cg.hip -> here): 300-cell cable
 // TT2006 FP64 133 -> 25 us; 64 x 64 x 16 TT2006 FP64 208 -> 69; 256 x 256
 // Mitchell-Schaeffer FP32+refine, per-cell rows, 173 -> 54; 490k-cell TT2006
-// FP32+refine with holes 321 -> 178; 492k-cell ORd FP32+refine, 27-point rows
-// per cell, 576 -> 405; 4M-cell batch TT2006 FP32+refine 945 -> 690.  What
+// FP32+refine with holes 321 -> 149; 492k-cell ORd FP32+refine, 27-point rows
+// per cell, 576 -> 345; 4M-cell batch TT2006 FP32+refine 945 -> 668.  What
 // bounds an iteration: 1.1 us of block sums, divisions and barriers on one
 // block, 3.1 us on 128 blocks (two trips of a word through the memory-side
 // cache), 6-14 us where a block holds 2,000-16,000 cells (LDS reads, and the
@@ -84,6 +84,7 @@ constexpr int kSumWords = 8;   // words of a block's sums: two each, to a line o
 constexpr int kSumBlocks = 8;  // blocks whose sums one load of a wave covers
 constexpr int kSumLoads = 16;  // such loads in flight together
 constexpr int kMaxSumWaves = 2;
+constexpr int kXcds = 8;
 
 // One halo cell of a tile.  Listed once per plan: found by every block in every
 // launch (a scan of its tile with divisions, an LDS counter) they took 8 of the
@@ -170,6 +171,7 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     int *flags;      // [0] a wait ended without its word, [1] halo count
 
     int tid, lane, wave;
+    int block;       // its tile and the place of its words
     int x0, y0, z0, ex, ey, ez, hx_, hy_, hz_;
     int dy, dz;      // neighbour strides in ext (0 along an axis of one cell)
     int nh;
@@ -202,7 +204,15 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         lane = tid & 63;
         wave = tid >> 6;
         const int nx = a.op64.nx, ny = a.op64.ny, nz = a.op64.nz;
-        const int bt = blockIdx.x, btx = bt % a.tx, bty = (bt / a.tx) % a.ty, btz = bt / (a.tx * a.ty);
+        // Blocks go to the eight XCDs in turn; an XCD's blocks take consecutive
+        // tiles, so that most neighbours are on one XCD and the lines that their
+        // rows, x and b share are in its L2 (490k-cell wedges, a step: 27-point
+        // rows per cell 415 -> 349 us, a table of rows 179 -> 149).
+        {
+            const int full = a.nblocks / kXcds, rest = a.nblocks % kXcds, x = blockIdx.x % kXcds;
+            block = x * full + (x < rest ? x : rest) + blockIdx.x / kXcds;
+        }
+        const int bt = block, btx = bt % a.tx, bty = (bt / a.tx) % a.ty, btz = bt / (a.tx * a.ty);
         x0 = btx * a.bx;
         y0 = bty * a.by;
         z0 = btz * a.bz;
@@ -261,9 +271,9 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             if constexpr(MIXED) fill_table(a.op32, rows, (float *)tab);
         }
         if(tid == 0) flags[0] = __hip_atomic_load(&a.st->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kResidentGoing;
-        nh = a.nblocks > 1 ? a.ncells[blockIdx.x] : 0;
+        nh = a.nblocks > 1 ? a.ncells[block] : 0;
         for(int i = tid; i < nh; i += T) {
-            const HaloCell h = a.cells[(size_t)blockIdx.x * a.halo + i];
+            const HaloCell h = a.cells[(size_t)block * a.halo + i];
             hword[i] = h.word;
             hext[i] = (uint16_t)h.ext;
         }
@@ -499,7 +509,7 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         u64 *S = a.sums + (size_t)(epoch & 1) * ((size_t)a.nblocks * kSumWords);
 #pragma unroll
         for(int q = 0; q < RPT; q++) {
-            if((edge >> q) & 1u) put_value(W + (size_t)kWords<T2> * ((size_t)blockIdx.x * (RPT * T) + local(q)), epoch, value(q));
+            if((edge >> q) & 1u) put_value(W + (size_t)kWords<T2> * ((size_t)block * (RPT * T) + local(q)), epoch, value(q));
             breathe<RPT == 32, 8>(q);
         }
         wave_sums(t);
@@ -522,7 +532,7 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
 #pragma unroll
             for(int i = 0; i < NW; i++) total += part[(tid >> 1) * NW + i];
             const u64 bits = (u64)__double_as_longlong(total);
-            word_store(&S[(size_t)blockIdx.x * kSumWords + tid], tagged(epoch, (tid & 1) ? (uint32_t)(bits >> 32) : (uint32_t)bits));
+            word_store(&S[(size_t)block * kSumWords + tid], tagged(epoch, (tid & 1) ? (uint32_t)(bits >> 32) : (uint32_t)bits));
         }
         return finish_exchange<T2>(t, store);
     }
@@ -637,7 +647,7 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     }
 
     __device__ __forceinline__ void note(int its, int outer, int inner, double err) {
-        if(blockIdx.x == 0 && tid == 0) {
+        if(block == 0 && tid == 0) {
             ResidentStatus *st = a.st;
             st->epoch = epoch;
             st->solves += 1;
@@ -697,11 +707,11 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
             for(int i = tid; i < nh; i += T) {
                 double xn;
                 if constexpr(MIXED) {
-                    if(sweep == 0) xn = a.x[a.cells[(size_t)blockIdx.x * a.halo + i].cell];
+                    if(sweep == 0) xn = a.x[a.cells[(size_t)block * a.halo + i].cell];
                     else xn = hx[i] + (double)hd[i];
                     hx[i] = xn;
                 } else {
-                    xn = a.x[a.cells[(size_t)blockIdx.x * a.halo + i].cell];
+                    xn = a.x[a.cells[(size_t)block * a.halo + i].cell];
                 }
                 ext64[hext[i]] = xn;
             }
