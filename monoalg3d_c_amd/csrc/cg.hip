@@ -316,7 +316,7 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
                                              double (&v)[Epi::NR]) {
     static_assert(9 * 27 <= kBlock && kMaskTable == kBlock, "one class-row coefficient or table entry per thread");
     // CM: 0 per-cell rows, 1 class table, 2 code table (7-point rows), 3 rows
-    // formed from neighbourhood masks (27-point)
+    // applied from neighbourhood masks (27-point)
     constexpr bool CLS = CM == 1;
     static_assert(CM != 2 || PAT == 7, "code tables hold 7-point rows");
     static_assert(CM != 3 || PAT == 27, "mask rows are 27-point rows");
