@@ -1559,7 +1559,7 @@ bool CgWorkspace::resident_begin(const OpView<double> &op64, const OpView<float>
         return false;
     }
     if(p.state != 1) return false;
-    if(resident_epochs + most * (unsigned)count > (1ull << 31)) {
+    if(!p.cleared || resident_epochs + most * (unsigned)count > (1ull << 31)) {
         if(resident_reset(rplan, 2, rst, s)) {
             *rc = -1;
             return false;

@@ -52,18 +52,21 @@ struct ResidentPlan {
     unsigned long long *sums = nullptr;   // partial sums of both parities
     void *cells = nullptr;                // halo cells of every tile
     int *ncells = nullptr;                // how many each tile has
+    bool cleared = false;        // words and sums hold no word of another run (resident_reset)
     uint64_t wait_ticks = 2000000;  // longest wait of a block for another: 20 ms of the 100 MHz clock
     size_t words_bytes = 0;
     size_t sums_bytes = 0;
 };
 
-// Decide the tiles for an operator and make the buffers (p->state).
+// Decide the tiles for an operator and make the buffers (p->state).  New ones
+// must be cleared before the first solve: memory that an earlier workspace gave
+// back holds words with the first epochs' numbers, which a reader would take.
 int resident_plan(ResidentPlan *p, const OpView<double> &op64, const OpView<float> *op32, const CgConfig &cfg);
 int resident_release(ResidentPlan *p);
 // Enqueues the solve; op32 null: FP64 CG.
 int resident_launch(const ResidentPlan &p, const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x,
                     const CgConfig &cfg, ResidentStatus *st, hipStream_t s);
 // Clears the exchange buffers and the epoch (and `stop`) on the stream.
-int resident_reset(const ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s);
+int resident_reset(ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s);
 
 }  // namespace mono

@@ -1029,11 +1029,12 @@ int resident_release(ResidentPlan *p) {
     return 0;
 }
 
-int resident_reset(const ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s) {
+int resident_reset(ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s) {
     for(int i = 0; i < nplans; i++) {
         if(i > 0 && plans[i].state != 1) continue;
         k_resident_reset<<<256, 256, 0, s>>>(plans[i].words, plans[i].words_bytes / sizeof(u64), plans[i].sums,
                                              plans[i].sums_bytes / sizeof(u64), st);
+        plans[i].cleared = true;
     }
     MONO_CHECK(hipGetLastError());
     return 0;
