@@ -138,7 +138,9 @@ constexpr bool holds_xb(bool mixed, int P, int rpt, bool table) {
 // are a table or stored per cell: from the smallest to the largest that fits,
 // no size was found where the launches of cg.hip take less time (1.1-6x over
 // domains of 300 to 4M cells).  Rows formed from neighbourhood masks, Jacobi
-// and CSR solves stay there.
+// and CSR solves stay there, and so do rows that reach across an axis of one
+// cell: a tile has no halo along such an axis (its neighbour strides are 0), so
+// their coefficients would multiply the cell itself.  Assembled rows are 0 there.
 //
 // Which shapes are built: a table in LDS with few cells per block or many;
 // rows per cell only where they are kept.
@@ -839,6 +841,7 @@ template <bool MIXED, class F> void with_kernel(int P, int threads, int rpt, boo
 
 // operator storage that the kernels read: 1 class table, 2 code table, 0 per-cell rows, -1 none
 template <typename TC> int storage(const OpView<TC> &op) {
+    if(op.thin) return -1;
     if(op.table) return 1;
     if(op.codes) return 2;
     return op.percell ? 0 : -1;

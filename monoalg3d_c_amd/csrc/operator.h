@@ -71,6 +71,7 @@ template <typename T> struct OpView {
     int64_t n;
     int pat;                    // pattern of table_int / percell (7, 19 or 27)
     int full_pat;               // class mode: pattern that covers every row, boundary rows too
+    bool thin;                  // some row reaches across an axis of one cell (to no neighbour)
     const T *table;             // class mode: [(z*9 + cy*3 + cx) * 27 + slot], else null
     const T *table_int;         // class mode: [z * pat + k] interior rows, else null
     const T *percell;           // per-cell mode: [k * n + cell], else null
@@ -108,6 +109,7 @@ struct Operator {
     int nint = 0;          // class mode: distinct slots of the interior rows
     int pat = 27;          // pattern of the interior rows (class mode) or of all rows (per-cell)
     int full_pat = 27;     // pattern that covers every row
+    bool thin = false;     // a non-zero slot along an axis of one cell
     bool class_mode = false;
     bool code_mode = false;
     bool mask32 = false;   // FP32 view in mask mode (the FP64 view keeps per-cell rows)

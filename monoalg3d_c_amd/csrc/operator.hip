@@ -639,6 +639,7 @@ static OpView<T> make_view(const Operator &o, const T *table, const T *tint, con
     v.n = o.n;
     v.pat = o.pat;
     v.full_pat = o.full_pat;
+    v.thin = o.thin;
     v.table = table;
     v.table_int = tint;
     v.percell = percell;
@@ -749,6 +750,9 @@ int build_operator(const AssemblyParams &p, const double *coef27, Operator *op, 
     for(int k = 0; k < 27; k++)
         if(k != 13 && (mask >> k) & 1u) slots.push_back(k);
     op->nslots = (int)slots.size();
+    op->thin = false;
+    for(int k : slots)
+        if((p.nx == 1 && k % 3 != 1) || (p.ny == 1 && k / 3 % 3 != 1) || (p.nz == 1 && k / 9 != 1)) op->thin = true;
     std::vector<int> bslots;  // the smallest pattern covering every row (per-cell storage order)
     const int pb = choose_pattern(slots, &bslots);
     op->full_pat = pb;
