@@ -1589,11 +1589,7 @@ int CgWorkspace::resident_enqueue(const OpView<double> &op64, const OpView<float
 int CgWorkspace::resident_finish(ResidentStatus *out, hipStream_t s) {
     MONO_CHECK(hipMemcpyAsync(host_rst, rst, sizeof(ResidentStatus), hipMemcpyDeviceToHost, s));
     MONO_CHECK(hipStreamSynchronize(s));
-    *out = *host_rst;
-    out->solves -= rst_seen.solves;
-    out->cg_total -= rst_seen.cg_total;
-    out->inner_total -= rst_seen.inner_total;
-    out->outer_total -= rst_seen.outer_total;
+    *out = resident_since(*host_rst, rst_seen);
     rst_seen = *host_rst;
     if(out->stop != kResidentGoing) {
         if(resident_reset(rplan, 2, rst, s)) return -1;

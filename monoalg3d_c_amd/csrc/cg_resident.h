@@ -6,30 +6,11 @@
 
 #include "mono_common.h"
 #include "operator.h"
+#include "resident_status.h"
 
 namespace mono {
 
 struct CgConfig;
-
-// Device record of the resident solves on one workspace.  The kernels of a
-// step do nothing while `stop` is set, so solves can be enqueued ahead of the
-// host's look at it.
-enum ResidentStop : int32_t {
-    kResidentGoing = 0,
-    kResidentNan = 1,      // the last solve ended with r.r = NaN (it is counted)
-    kResidentTimeout = 2,  // a block waited too long for another: the solve is not done
-};
-struct ResidentStatus {
-    int32_t stop;
-    uint32_t epoch;        // exchanges done so far on this workspace
-    int64_t solves;        // solves completed
-    int64_t cg_total;      // sum of the reference's iteration counts
-    int64_t inner_total;   // CG iterations run
-    int64_t outer_total;   // outer sweeps
-    int32_t last_its;
-    int32_t last_outer;
-    double last_err;
-};
 
 // One block's share of the box and how many blocks there are.
 struct ResidentGeom {
@@ -66,7 +47,7 @@ int resident_release(ResidentPlan *p);
 // Enqueues the solve; op32 null: FP64 CG.
 int resident_launch(const ResidentPlan &p, const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x,
                     const CgConfig &cfg, ResidentStatus *st, hipStream_t s);
-// Clears the exchange buffers and the epoch (and `stop`) on the stream.
+// Clears the exchange buffers, the epoch, `stop` and `left` on the stream.
 int resident_reset(ResidentPlan *plans, int nplans, ResidentStatus *st, hipStream_t s);
 
 }  // namespace mono

@@ -376,19 +376,25 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
     template <int N> __device__ __forceinline__ void await(const u64 *const (&p)[N], uint32_t (&h)[N], bool &bad) {
         u64 v[N];
         u64 began = 0;
+        bool last = bad;  // an earlier wait of this exchange has ended without its words
         for(int n = 1;; n++) {
             bool all = true;
 #pragma unroll
             for(int k = 0; k < N; k++) v[k] = word_load(p[k]);
 #pragma unroll
             for(int k = 0; k < N; k++) all &= (uint32_t)(v[k] >> 32) == epoch;
-            if(all || bad) break;
+            if(all) break;
+            if(last) {
+                bad = true;
+                break;
+            }
             if((n & 63) == 0 || a.wait_ticks == 0) {
                 const u64 now = wall_clock64();
                 if(began == 0) began = now;
-                // (one more look at the words follows)
+                // (one more look at the words follows, and counts: a wave that was
+                // held up itself finds them there)
                 if(now - began >= a.wait_ticks || __hip_atomic_load(&a.st->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kResidentTimeout)
-                    bad = true;
+                    last = true;
             }
         }
 #pragma unroll
@@ -663,7 +669,10 @@ template <bool MIXED, int P, int T, int RPT, bool TABLE> struct Resident {
         }
     }
     __device__ __forceinline__ void timed_out() {
-        if(tid == 0) __hip_atomic_store(&a.st->stop, (int32_t)kResidentTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if(tid == 0) {
+            __hip_atomic_fetch_max(&a.st->left, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a.st->stop, (int32_t)kResidentTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 
     __device__ __forceinline__ void run(char *lds) {
@@ -807,6 +816,7 @@ __global__ void k_resident_reset(u64 *words, size_t nwords, u64 *sums, size_t ns
     for(size_t k = i; k < nsums; k += step) sums[k] = 0;
     if(i == 0) {
         st->epoch = 0;
+        st->left = 0;
         st->stop = kResidentGoing;
     }
 }
