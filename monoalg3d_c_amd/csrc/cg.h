@@ -157,8 +157,7 @@ class CgWorkspace {
     ResidentStatus rst_seen{};           // the record at the last resident_finish
     uint64_t resident_epochs = 0;     // bound on the exchanges since the last reset
     bool use_resident = true;         // MONO_RESIDENT=0 in the environment at init: never
-    int resident_pause = 0;           // after a time-out: solves left to the kernels of cg.hip
-    int resident_backoff = 0;
+    ResidentPause resident_pause;
 
   private:
     int solve_one_resident(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x, const CgConfig &cfg,

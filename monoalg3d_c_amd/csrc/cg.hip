@@ -1546,10 +1546,7 @@ bool CgWorkspace::resident_begin(const OpView<double> &op64, const OpView<float>
                                  int *rc) {
     *rc = 0;
     if(!rst || !use_resident || cfg.jacobi || cfg.poll_chunk > 0 || count < 1) return false;
-    if(resident_pause > 0) {
-        resident_pause--;
-        return false;
-    }
+    if(resident_pause.left > 0) return false;
     // exchanges a solve may need; their 32-bit numbers start again long before they run out
     const uint64_t most = op32 ? ((uint64_t)cfg.max_its + 3) * ((uint64_t)cfg.max_outer + 1) : (uint64_t)cfg.max_its + 2;
     if(cfg.max_its < 0 || cfg.max_outer < 0 || most > (1ull << 30) / (unsigned)count) return false;
@@ -1594,13 +1591,9 @@ int CgWorkspace::resident_finish(ResidentStatus *out, hipStream_t s) {
     if(out->stop != kResidentGoing) {
         if(resident_reset(rplan, 2, rst, s)) return -1;
         resident_epochs = 0;
-        if(out->stop == kResidentTimeout) {
-            // the chip is shared with launches of the same kind: leave it to
-            // the others for a while, each time for longer
-            resident_backoff = resident_backoff < 1024 ? 4 * resident_backoff + 16 : resident_backoff;
-            resident_pause = resident_backoff;
-        }
     }
+    resident_pause.solved(out->solves);
+    if(out->stop == kResidentTimeout) resident_pause.timed_out();
     return 0;
 }
 
@@ -1628,6 +1621,7 @@ int CgWorkspace::solve_fp64(const OpView<double> &op, const double *b, double *x
         if(rc <= 0) return rc;
     }
     if(rrc) return -1;
+    resident_pause.spent();
     int nres = 0;
     auto iterations = [&](int k0, int count) -> int { return fp64_launches(op, b, x, cfg, k0, count, nres, s); };
     // the last solve's iteration count includes the kernel that detected
@@ -1670,6 +1664,7 @@ int CgWorkspace::solve_mixed(const OpView<double> &op64, const OpView<float> &op
         if(rc <= 0) return rc;
     }
     if(rrc) return -1;
+    resident_pause.spent();
     float *pb[2] = {p32, p32b};
     int inner_total = 0, corrections = 0;
     int chunk0 = last_inner > 2 ? last_inner + 1 : 4;

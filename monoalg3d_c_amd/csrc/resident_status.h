@@ -53,4 +53,28 @@ inline ResidentStatus resident_since(const ResidentStatus &now, const ResidentSt
     return r;
 }
 
+// After a time-out the chip is shared with launches of the same kind: the next
+// solves are left to the kernels of cg.hip, more of them after each further
+// time-out (16, 80, 336, then 1360).  As many solves in one launch without a
+// time-out as the last pause was long end the lengthening.
+struct ResidentPause {
+    int left = 0;      // solves still to be left to the other kernels
+    int length = 0;    // of the last pause
+    int64_t good = 0;  // solves in one launch since the last time-out
+
+    void timed_out() {
+        length = length < 1024 ? 4 * length + 16 : length;
+        left = length;
+        good = 0;
+    }
+    void solved(int64_t n) {
+        good += n;
+        if(good >= length) length = 0;
+    }
+    // a solve was done by the other kernels
+    void spent() {
+        if(left > 0) left--;
+    }
+};
+
 }  // namespace mono
