@@ -172,6 +172,12 @@ int mono_tissue_set_timing(mono_tissue *t, int on);
  * and how many such graphs it recorded.  Recording is opt-in: MONO_GRAPH=1 in
  * the environment when the tissue is created. */
 int mono_tissue_graph_counts(const mono_tissue *t, int64_t *launches, int64_t *captures);
+/* No reference counterpart (diagnostic): how many of the tissue's steps had
+ * their diffusion solve done in one launch, and how many such solves ended
+ * because a block waited too long for another (those steps are solved again,
+ * in several launches).  MONO_RESIDENT=0 in the environment when the tissue is
+ * created: none are done in one launch. */
+int mono_tissue_resident_counts(const mono_tissue *t, int64_t *solves, int64_t *timeouts);
 /* device pointers for zero-copy consumers: v (FP64, n), sv (neq rows of
  * `pitch` elements, FP64 or FP32 by precision), b (FP64, n) */
 int mono_tissue_device_ptrs(mono_tissue *t, void **v, void **sv, size_t *pitch, void **b);

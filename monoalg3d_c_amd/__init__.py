@@ -214,6 +214,12 @@ class Tissue:
         check(lib().mono_tissue_graph_counts(self._h, C.byref(launches), C.byref(captures)), "mono_tissue_graph_counts")
         return launches.value, captures.value
 
+    def resident_counts(self) -> tuple:
+        """(steps whose solve was one launch, such solves that gave up waiting and were done again otherwise)."""
+        solves, timeouts = C.c_int64(), C.c_int64()
+        check(lib().mono_tissue_resident_counts(self._h, C.byref(solves), C.byref(timeouts)), "mono_tissue_resident_counts")
+        return solves.value, timeouts.value
+
     @property
     def v(self) -> np.ndarray:
         out = np.empty(self.n, np.float64)

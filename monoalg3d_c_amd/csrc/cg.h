@@ -158,6 +158,8 @@ class CgWorkspace {
     uint64_t resident_epochs = 0;     // bound on the exchanges since the last reset
     bool use_resident = true;         // MONO_RESIDENT=0 in the environment at init: never
     ResidentPause resident_pause;
+    int64_t resident_solves = 0;    // statistics
+    int64_t resident_timeouts = 0;
 
   private:
     int solve_one_resident(const OpView<double> &op64, const OpView<float> *op32, const double *b, double *x, const CgConfig &cfg,

@@ -1592,8 +1592,12 @@ int CgWorkspace::resident_finish(ResidentStatus *out, hipStream_t s) {
         if(resident_reset(rplan, 2, rst, s)) return -1;
         resident_epochs = 0;
     }
+    resident_solves += out->solves;
     resident_pause.solved(out->solves);
-    if(out->stop == kResidentTimeout) resident_pause.timed_out();
+    if(out->stop == kResidentTimeout) {
+        resident_timeouts++;
+        resident_pause.timed_out();
+    }
     return 0;
 }
 

@@ -496,6 +496,13 @@ int mono_tissue_graph_counts(const mono_tissue *t, int64_t *launches, int64_t *c
     return 0;
 }
 
+int mono_tissue_resident_counts(const mono_tissue *t, int64_t *solves, int64_t *timeouts) {
+    if(!t) return -1;
+    if(solves) *solves = t->cg.resident_solves;
+    if(timeouts) *timeouts = t->cg.resident_timeouts;
+    return 0;
+}
+
 static int launch_ionic(mono_tissue *t, double stim_amp, int block) {
     const mono_tissue_desc &d = t->d;
     if(d.precision == MONO_FP64) {
