@@ -284,9 +284,9 @@ __host__ __device__ __forceinline__ void mask_assemble_fast(const T (&h)[kNDir],
 }
 
 // FAST: the flux sigmas by mask_flux_fast and the coefficients by
-// mask_assemble_fast (what a kernel that needs the coefficients themselves
-// would use; checked on the host); otherwise the operations of k_assemble in
-// its order.
+// mask_assemble_fast (no kernel needs the coefficients themselves any more:
+// only the host test of the rows calls this form); otherwise the operations of
+// k_assemble in its order.
 template <typename T, bool FAST = false>
 __host__ __device__ __forceinline__ void mask_aniso_row(uint32_t m, const T (&tz)[3][6], T dx, T dy, T dz, T alpha, T (&row)[27]) {
 #pragma unroll

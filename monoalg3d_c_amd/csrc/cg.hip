@@ -386,7 +386,8 @@ __device__ __forceinline__ void tile_segment(const OpView<TC> &op, const TileGeo
         }
     };
     // mask mode: the weights of a plane's layer are staged in LDS, one plane
-    // ahead; class mode: likewise the 9 class rows of a plane (27 slots each), for tiles on an x or y face and on the boundary planes
+    // ahead; class mode: likewise the 9 class rows of a plane (27 slots each),
+    // for tiles on an x or y face and on the boundary planes
     const bool face_xy = CLS && (x0 < g.lo[0] || x0 + kTX - 1 > g.hi[0] || y0 < g.lo[1] || y0 + kTY - 1 > g.hi[1]);
     auto need_rows = [&](int z) { return CLS && (face_xy || z < g.lo[2] || z > g.hi[2]); };
     TC rrow = TC(0);

@@ -24,10 +24,10 @@
 // per iteration carries them and the sums.
 //
 // Measured (one MI355X, whole steps, launches of cg.hip -> here): 300-cell cable
-// TT2006 FP64 133 -> 25 us; 64 x 64 x 16 TT2006 FP64 208 -> 69; 256 x 256
-// Mitchell-Schaeffer FP32+refine, per-cell rows, 173 -> 54; 490k-cell TT2006
-// FP32+refine with holes 321 -> 149; 492k-cell ORd FP32+refine, 27-point rows
-// per cell, 576 -> 345; 4M-cell batch TT2006 FP32+refine 945 -> 668.  What
+// TT2006 FP64 129 -> 25 us; 64 x 64 x 16 TT2006 FP64 210 -> 66; 256 x 256
+// Mitchell-Schaeffer FP32+refine, per-cell rows, 177 -> 53; 490k-cell TT2006
+// FP32+refine with holes 323 -> 145; 492k-cell ORd FP32+refine, 27-point rows
+// per cell, 585 -> 343; 4M-cell batch TT2006 FP32+refine 942 -> 680.  What
 // bounds an iteration: 1.1 us of block sums, divisions and barriers on one
 // block, 3.1 us on 128 blocks (two trips of a word through the memory-side
 // cache), 6-14 us where a block holds 2,000-16,000 cells (LDS reads, and the
@@ -122,10 +122,15 @@ struct Shape {
 };
 constexpr Shape kShapes[] = {{256, 1}, {256, 2}, {512, 2}, {512, 4}, {512, 8}, {512, 32}};
 
-// Whether the rows of own cells are kept in registers for the whole solve
-// (rows stored per cell, where they fit): read again in every iteration they
-// would come from the memory-side cache at a latency that these few waves
-// cannot hide (27-point rows of 492k cells: 40 us an iteration).
+// Whether the rows of own cells are kept for the whole solve (rows stored per
+// cell): read again in every iteration they would come from the memory-side
+// cache at a latency that these few waves cannot hide (27-point rows of 492k
+// cells: 40 us an iteration, 8 us kept).  The bound is on the coefficients
+// alone: up to 64 or 112 registers a thread.  In the largest such shapes the
+// compiler then spills other values, or some of the rows, to scratch: 77
+// registers of FP64 7-point rows at 512 x 8, 36 of mixed 27-point rows at
+// 512 x 4, 24 of mixed 7-point rows at 512 x 8, 7 of mixed 19-point rows at 512 x 4,
+// 2 of FP64 27-point rows at 512 x 2.
 constexpr bool keeps_rows(bool mixed, int P, int T, int rpt, bool table) {
     return !table && rpt * P * (mixed ? 1 : 2) <= (T == 512 ? 112 : 64);
 }

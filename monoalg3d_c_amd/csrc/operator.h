@@ -92,7 +92,10 @@ template <typename T> struct OpView {
 // 4-byte mask per cell and its kernels apply each row as sums of masked
 // differences (aniso_row.h) instead of reading 27 stored coefficients; enabled
 // only after rows formed from the masks in FP64 reproduced every assembled
-// row bit for bit.  MONO_MASK_ROWS=0 keeps the stored FP32 rows.
+// row bit for bit.  That check is of the masks and of the rule; the product
+// itself and its layer tables are compared with the oracle's rows by a host
+// test and with stored rows by a GPU test.  MONO_MASK_ROWS=0 keeps the stored
+// FP32 rows.
 //
 // Code mode: when every 7-point row is fixed by which of its six neighbours
 // exist and are active (a uniform isotropic tensor on a box with inactive

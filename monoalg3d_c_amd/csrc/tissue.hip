@@ -567,10 +567,6 @@ static int launch_ionic(mono_tissue *t, double stim_amp, int block) {
     return 0;
 }
 
-// The block size for this step's ionic launch from the tuner: the previous
-// trial's time is read back (its launch finished within the previous step's
-// solve, which waited on the device), then the next candidate, or the fastest
-// once every candidate has run twice after the first step.
 // Partial ||b_i||^2 of one work item (one wave): up to kInstCols cells of one
 // row of instance i's bounding box (a row: one (y, z) line of the box), all
 // loads issued at once, summed in a fixed order into part[item]
@@ -637,6 +633,10 @@ static int launch_instance_tolerance(mono_tissue *t) {
     return 0;
 }
 
+// The block size for this step's ionic launch from the tuner: the previous
+// trial's time is read back (waiting for its launch, where steps are enqueued
+// ahead of the device), then the next candidate, or the fastest once every
+// candidate has run twice after the first step.
 static int tuned_block(mono_tissue *t, bool &timed) {
     auto &u = t->tune;
     timed = false;
